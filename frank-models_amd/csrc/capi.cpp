@@ -308,7 +308,7 @@ BlockLayout block_layout(int64_t T, int64_t E, int64_t k, int64_t H, int64_t F, 
                                                        static_cast<int>(E), static_cast<int>(k), act),
                            router_prefill_scratch_bytes(static_cast<int>(T), static_cast<int>(H),
                                                         static_cast<int>(E), static_cast<int>(k), act));
-  off += align_up(L.rpart_bytes);
+  if (act != FMOE_F32) off += align_up(L.rpart_bytes);
   L.h_dtype = act;
   L.h = off;
   off += align_up(static_cast<size_t>(n) * F * dtype_bytes(L.h_dtype));
@@ -316,7 +316,14 @@ BlockLayout block_layout(int64_t T, int64_t E, int64_t k, int64_t H, int64_t F, 
   L.y_part_elems = n * H;
   L.y_parts = (n > 0 && H > 0 && F > 0) ? gemm_tiled256_ksplit(down_shape(T, E, k, H, F, act, wdt)) : 1;
   L.y = off;
-  off += align_up(static_cast<size_t>(n) * H * dtype_bytes(L.y_dtype) * L.y_parts);
+  const size_t y_bytes = align_up(static_cast<size_t>(n) * H * dtype_bytes(L.y_dtype) * L.y_parts);
+  off += y_bytes;
+  // fp32 batches keep the partial router logits in the y rows, which the
+  // down projection writes long after the top-k has read them.
+  if (act == FMOE_F32) {
+    L.rpart = L.y;
+    L.rpart_bytes = L.rpart_bytes <= y_bytes ? L.rpart_bytes : 0;
+  }
   // Prefill-sized bf16 batches: room for the token rows gathered into expert
   // order, K-blocked, so the gate/up GEMM reads whole cache lines.
   const bool prefill = act == FMOE_BF16 && n > 8 * E;
@@ -862,6 +869,19 @@ int run_linear(const void* x, int64_t K, const void* packed, const float* scales
     FMOE_HIP(launch_gemm_stream(g, s));
     g_last_path = FMOE_PATH_STREAM;
     *nsplit = g.ksplit;
+    return FMOE_OK;
+  }
+  // fp32: the same split, for about two blocks per CU and at least 4 stages
+  // of 32 inputs per piece.
+  if (g_path.load(std::memory_order_relaxed) == FMOE_PATH_AUTO && gemm_f32_supported(g)) {
+    const int64_t tiles = static_cast<int64_t>((B + 63) / 64) * ((N + 127) / 128);
+    int ks = 1;
+    while (ks * 2 <= kLinearMaxSplit && tiles * ks * 2 <= 512 && K / 32 / (ks * 2) >= 4) ks *= 2;
+    g.ksplit = ks;
+    g.split_stride = static_cast<int64_t>(B) * N;
+    FMOE_HIP(launch_gemm_f32(g, s));
+    g_last_path = FMOE_PATH_TILED;
+    *nsplit = ks;
     return FMOE_OK;
   }
   g.order = order;

@@ -1098,6 +1098,7 @@ bool gemm_stream_supported(const GroupedGemmArgs& g) {
 }
 
 int resolve_tiled_variant(const GroupedGemmArgs& g, int variant) {
+  if (gemm_f32_supported(g)) return TILED_F32;
   const bool large_ok = gemm_tiled256_supported(g);
   const bool small_ok = g.epi <= EPI_SCATTER_WEIGHTED && mfma_common_ok(g) && grouping_ok(g, false) &&
                         g.K % kBK == 0 && g.K > 0 && g.ksplit == 1;
@@ -1113,6 +1114,7 @@ int resolve_tiled_variant(const GroupedGemmArgs& g, int variant) {
 hipError_t launch_gemm_tiled(const GroupedGemmArgs& g, hipStream_t s, int variant) {
   const int v = resolve_tiled_variant(g, variant);
   if (v == TILED_256) return launch_gemm_tiled256(g, s);
+  if (v == TILED_F32) return launch_gemm_f32(g, s);
   if (v != TILED_128) return hipErrorNotSupported;
   if (g.n_assign == 0 || g.N == 0) return hipSuccess;
   // 96 KiB of dynamic LDS per block (gfx950 has 160 KiB per CU); set once per process.

@@ -192,8 +192,8 @@ hipError_t launch_router(const void* x, const void* wr, int n_tokens, int n_embd
                          int n_expert, int k, bool normalize, int dtype, int* ids,
                          float* weights, hipStream_t stream);
 
-// Decode-sized batches (bf16, n_tokens <= kDecodeMaxTokens, n_expert <= 256,
-// k <= 16): router logits split over many blocks into `part`
+// Decode-sized batches (bf16, or fp32 with n_embd % 16 == 0; n_tokens <=
+// kDecodeMaxTokens, n_expert <= 256, k <= 16): router logits split over many blocks into `part`
 // (router_decode_scratch_bytes, 0 when the shape does not qualify), then one
 // block runs softmax + top-k and the permutation (ids, weights, order,
 // offsets, err_count as launch_router + launch_permute write them); above 64
@@ -214,8 +214,8 @@ hipError_t launch_router_split_logits(const void* x, const void* wr, int n_token
 int router_decode_splits(int n_embd);
 
 // Prefill batches (bf16, n_tokens > kDecodeMaxTokens, 32 < n_expert <= 128,
-// n_embd % 128 == 0, k <= 16): router logits over 64-token tiles and
-// ranges of the hidden axis into `part` (router_prefill_scratch_bytes, 0
+// n_embd % 128 == 0, k <= 16; or fp32, n_expert <= 256, n_embd % 16 == 0):
+// router logits over 64-token tiles (fp32: 16 tokens x 16 experts) and ranges of the hidden axis into `part` (router_prefill_scratch_bytes, 0
 // when the shape does not qualify), then softmax + top-k summing the ranges
 // in order (ids, weights as launch_router writes them).
 // hipErrorNotSupported when the inputs do not qualify.
@@ -254,9 +254,10 @@ hipError_t launch_pack(const void* src, int src_dtype, const float* src_scales,
 hipError_t launch_gemm_generic(const GroupedGemmArgs& g, hipStream_t stream);
 // Returns hipErrorNotSupported when the shape or dtype is outside what the
 // MFMA kernels handle; the caller then uses the generic kernel.
-enum TiledVariant { TILED_AUTO = 0, TILED_128 = 1, TILED_256 = 2 };
+enum TiledVariant { TILED_AUTO = 0, TILED_128 = 1, TILED_256 = 2, TILED_F32 = 3 };
 // The tiled kernel that `variant` resolves to for g (TILED_AUTO picks the
-// 256x256-tile kernel wherever it applies), or -1 if none applies.
+// 256x256-tile kernel wherever it applies; fp32 operands resolve to
+// TILED_F32), or -1 if none applies.
 int resolve_tiled_variant(const GroupedGemmArgs& g, int variant);
 hipError_t launch_gemm_tiled(const GroupedGemmArgs& g, hipStream_t stream, int variant);
 hipError_t launch_gemm_stream(const GroupedGemmArgs& g, hipStream_t stream);
@@ -273,6 +274,11 @@ bool gemm_stream_supported(const GroupedGemmArgs& g);
 // Whether the streaming gate/up GEMM takes g with its routing (g.rp set):
 // the shape qualifies and the grid fits one round of resident blocks.
 bool gemm_stream_routed_ok(const GroupedGemmArgs& g);
+// fp32 activations and weights on the fp32 matrix instruction (gemm_f32.hip);
+// takes a K split (EPI_SCATTER) and, for one expert's rows in order, no
+// grouping arrays, as the streaming kernel does.
+bool gemm_f32_supported(const GroupedGemmArgs& g);
+hipError_t launch_gemm_f32(const GroupedGemmArgs& g, hipStream_t stream);
 // 256x256-tile bf16 kernel (gemm_tiled256.hip); launch_gemm_tiled uses it
 // when it applies.
 bool gemm_tiled256_supported(const GroupedGemmArgs& g);

@@ -19,7 +19,11 @@
 //     permutation: one wave up to 4 tokens (router_topk_permute_wave_kernel);
 //     above 64 experts and 32 tokens router_part_topk_kernel over blocks,
 //     then the permutation's own launch);
-//   * router_simt_kernel: fp32 and the shapes above that none takes.
+//   * router_split_logits_f32_kernel: the same split for fp32, at any batch
+//     size (router_part_topk_kernel above 64 tokens);
+//   * router_mfma_f32_kernel: fp32, up to 128 experts, where there is no room
+//     for partial logits (fmoe_router has no workspace) or k > 16;
+//   * router_simt_kernel: the shapes above that none takes.
 // Softmax + top-k run four tokens per wave (16 lanes each, DPP row
 // reductions) for k <= 16, or one token per wave over its 64 lanes.
 #include "common.h"
@@ -34,6 +38,7 @@ constexpr int kTok = 16;
 constexpr int kThreads = 256;
 constexpr int kMaxExpert = 256;    // lanes hold up to 4 experts each
 constexpr int kMfmaMaxExpert = 128;
+constexpr int kF32MaxEmbd = 1 << 20;  // fp32 kernels: 32-bit element offsets, grid z of the split
 
 // Softmax + top-k + optional renormalisation of token t, whose logits are
 // lg[0 .. n_expert), by one wave with the expert axis spread over its lanes.
@@ -230,6 +235,81 @@ __global__ __launch_bounds__(kMfmaThreads) void router_mfma_bf16_kernel(
         if (c < n_chunks)
           acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av[d]),
                                                            __builtin_bit_cast(bf16x8_t, bv[d][c]), acc[c], 0, 0, 0);
+  }
+  // D[token][expert]: lane holds expert (lane & 15), tokens 4*(lane>>4)+i.
+  float* mine = part + wave * kTok * ld;
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    if (c < n_chunks) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mine[((lane >> 4) * 4 + i) * ld + c * 16 + (lane & 15)] = acc[c][i];
+    }
+  }
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < kTok * n_expert; idx += kMfmaThreads) {
+    const int tt = idx / n_expert;
+    const int e = idx - tt * n_expert;
+    float v = part[tt * ld + e];
+    for (int w = 1; w < kMfmaWaves; ++w) v += part[(w * kTok + tt) * ld + e];
+    logits[tt * ld + e] = v;
+  }
+  __syncthreads();
+  softmax_topk<kMfmaMaxExpert / 16>(logits, ld, tok0, n_tokens, n_expert, k, normalize != 0, ids, weights,
+                                    kMfmaWaves);
+}
+
+// fp32 inputs with n_embd % 16 == 0 and n_expert <= 128: the same block on
+// v_mfma_f32_16x16x4_f32 (fp32 products and sums).  A trip is 16 hidden
+// columns: lane l loads the 16 bytes of row l % 16 at columns 4 (l / 16) and
+// MFMA j multiplies element j of both operands, so each trip adds its 16
+// products over 4 instructions.
+// D: trips loaded before the first MFMA, as many as the 128 registers of a
+// 16-wave block hold.
+template <int NCH>
+__global__ __launch_bounds__(kMfmaThreads) void router_mfma_f32_kernel(
+    const float* __restrict__ x, const float* __restrict__ wr, int n_tokens, int n_embd, int n_expert, int k,
+    int normalize, int* __restrict__ ids, float* __restrict__ weights) {
+  extern __shared__ float part[];  // [kMfmaWaves][kTok][ld], then logits [kTok][ld]
+  const int ld = ((n_expert + 15) / 16) * 16 + 1;
+  float* logits = part + kMfmaWaves * kTok * ld;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int tok0 = blockIdx.x * kTok;
+  const int n_chunks = (n_expert + 15) / 16;
+  const int row = lane & 15;
+  const int kofs = (lane >> 4) * 4;
+
+  // Rows past the batch or the expert count read the last valid one (their
+  // logits are never used).
+  const float* xrow = x + static_cast<int64_t>(min(tok0 + row, n_tokens - 1)) * n_embd + kofs;
+  uint32_t wrow[NCH];  // element offsets (n_embd <= kF32MaxEmbd)
+#pragma unroll
+  for (int c = 0; c < NCH; ++c)
+    wrow[c] = static_cast<uint32_t>(min(c * 16 + row, n_expert - 1)) * static_cast<uint32_t>(n_embd) + kofs;
+  f32x4_t acc[NCH];
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) acc[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const f32x4_t zero{0.f, 0.f, 0.f, 0.f};
+  constexpr int kStep = kMfmaWaves * 16;
+  constexpr int D = NCH == 1 ? 8 : NCH == 2 ? 6 : NCH <= 4 ? 3 : 1;
+  for (int h0 = wave * 16; h0 < n_embd; h0 += D * kStep) {
+    f32x4_t av[D], bv[D][NCH];
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int h = h0 + d * kStep;
+      const bool in = h < n_embd;
+      av[d] = in ? *reinterpret_cast<const f32x4_t*>(xrow + h) : zero;
+#pragma unroll
+      for (int c = 0; c < NCH; ++c)
+        bv[d][c] = in ? *reinterpret_cast<const f32x4_t*>(wr + (wrow[c] + h)) : zero;
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int c = 0; c < NCH; ++c)
+            acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[d][j], bv[d][c][j], acc[c], 0, 0, 0);
   }
   // D[token][expert]: lane holds expert (lane & 15), tokens 4*(lane>>4)+i.
   float* mine = part + wave * kTok * ld;
@@ -511,6 +591,53 @@ __global__ __launch_bounds__(kSplitWaves * kWave) void router_split_logits_kerne
   }
 }
 
+// The same for fp32 inputs (n_embd % 16 == 0) on v_mfma_f32_16x16x4_f32, any
+// batch size: a wave's 128 columns are 8 trips of 16, all loaded before the
+// first MFMA.  One block per 16 tokens that streamed the whole router matrix
+// (router_mfma_f32_kernel) is bound by its one CU's loads: 24.9 us for 1
+// token and 30.0 us for 500 at 64 experts x 2048 columns.
+__global__ __launch_bounds__(kSplitWaves * kWave) void router_split_logits_f32_kernel(
+    const float* __restrict__ x, const float* __restrict__ wr, int n_tokens, int n_embd, int n_expert,
+    float* __restrict__ part) {
+  __shared__ f32x4_t red[kSplitWaves][kWave];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = threadIdx.x / kWave;
+  const int row = lane & 15, kofs = (lane >> 4) * 4;
+  const int t = min(static_cast<int>(blockIdx.x) * 16 + row, n_tokens - 1);   // rows past the end repeat
+  const int e = min(static_cast<int>(blockIdx.y) * 16 + row, n_expert - 1);   // the last token / expert
+  const float* xr = x + static_cast<int64_t>(t) * n_embd + kofs;
+  const float* wrow = wr + static_cast<int64_t>(e) * n_embd + kofs;
+  const int h0 = static_cast<int>(blockIdx.z) * kSplitCols + wave * 128;
+  const f32x4_t zero{0.f, 0.f, 0.f, 0.f};
+  f32x4_t a[8], b[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int h = h0 + 16 * j;
+    a[j] = h < n_embd ? *reinterpret_cast<const f32x4_t*>(xr + h) : zero;
+    b[j] = h < n_embd ? *reinterpret_cast<const f32x4_t*>(wrow + h) : zero;
+  }
+  f32x4_t acc = zero;
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][i], b[j][i], acc, 0, 0, 0);
+  red[wave][lane] = acc;
+  __syncthreads();
+  if (wave == 0) {
+    f32x4_t v = red[0][lane];
+#pragma unroll
+    for (int w = 1; w < kSplitWaves; ++w) v += red[w][lane];
+    // D[token][expert]: lane holds expert (lane & 15), tokens 4*(lane>>4)+i.
+    const int ee = static_cast<int>(blockIdx.y) * 16 + row;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int tt = static_cast<int>(blockIdx.x) * 16 + (lane >> 4) * 4 + i;
+      if (tt < n_tokens && ee < n_expert)
+        part[(static_cast<int64_t>(blockIdx.z) * n_tokens + tt) * n_expert + ee] = v[i];
+    }
+  }
+}
+
 // One block: logits = the splits' partials summed in split order, softmax +
 // top-k four tokens per wave (n_expert <= 16 NV), then the permutation of the
 // k * T slot-major ids, read back from an LDS copy.  The partials of kSumU
@@ -613,6 +740,17 @@ void launch_router_mfma(const void* x, const void* wr, int n_tokens, int n_embd,
                      n_expert, k, normalize ? 1 : 0, ids, weights);
 }
 
+template <int NCH>
+void launch_router_mfma_f32(const void* x, const void* wr, int n_tokens, int n_embd, int n_expert, int k,
+                            bool normalize, int* ids, float* weights, size_t lds, hipStream_t stream) {
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(router_mfma_f32_kernel<NCH>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  (void)attr;
+  hipLaunchKernelGGL((router_mfma_f32_kernel<NCH>), dim3((n_tokens + kTok - 1) / kTok), dim3(kMfmaThreads), lds,
+                     stream, static_cast<const float*>(x), static_cast<const float*>(wr), n_tokens, n_embd, n_expert,
+                     k, normalize ? 1 : 0, ids, weights);
+}
+
 template <int NCP, int TT>
 void launch_router_tile(const bf16_t* x, const bf16_t* wr, int n_tokens, int n_embd, int n_expert, int k,
                         bool normalize, int n_split, int stages_per_range, int* ids, float* weights, float* part,
@@ -656,6 +794,20 @@ hipError_t launch_router(const void* x, const void* wr, int n_tokens, int n_embd
     else
       launch_router_mfma<kMfmaMaxExpert / 16>(x, wr, n_tokens, n_embd, n_expert, k, normalize, ids, weights, lds,
                                               stream);
+  } else if (dtype == DT_F32 && n_embd % 16 == 0 && n_embd <= kF32MaxEmbd && n_expert <= kMfmaMaxExpert &&
+             aligned) {
+    const int n_chunks = (n_expert + 15) / 16;
+    const int ld = n_chunks * 16 + 1;
+    const size_t lds = static_cast<size_t>(kMfmaWaves + 1) * kTok * ld * sizeof(float);
+    if (n_chunks == 1)
+      launch_router_mfma_f32<1>(x, wr, n_tokens, n_embd, n_expert, k, normalize, ids, weights, lds, stream);
+    else if (n_chunks == 2)
+      launch_router_mfma_f32<2>(x, wr, n_tokens, n_embd, n_expert, k, normalize, ids, weights, lds, stream);
+    else if (n_chunks <= 4)
+      launch_router_mfma_f32<4>(x, wr, n_tokens, n_embd, n_expert, k, normalize, ids, weights, lds, stream);
+    else
+      launch_router_mfma_f32<kMfmaMaxExpert / 16>(x, wr, n_tokens, n_embd, n_expert, k, normalize, ids, weights, lds,
+                                                  stream);
   } else {
     const size_t lds = static_cast<size_t>(kTok) * (n_expert + 1) * sizeof(float);
     if (dtype == DT_BF16) {
@@ -675,7 +827,40 @@ hipError_t launch_router(const void* x, const void* wr, int n_tokens, int n_embd
 
 namespace fmoe {
 
+namespace {
+
+// fp32 batches of any size whose logits are split over blocks.
+bool f32_split_ok(int n_tokens, int n_embd, int n_expert, int k) {
+  return n_tokens > 0 && n_embd % 16 == 0 && n_embd <= kF32MaxEmbd && n_expert > 0 && n_expert <= kMaxExpert &&
+         k > 0 && k <= 16 && k <= n_expert;
+}
+
+hipError_t launch_part_topk(const float* part, int n_split, int n_tokens, int n_expert, int k, bool normalize,
+                            int* ids, float* weights, hipStream_t stream) {
+  const dim3 grid((n_tokens + 4 * kPartWaves - 1) / (4 * kPartWaves));
+  if (n_expert <= 64)
+    hipLaunchKernelGGL(router_part_topk_kernel<4>, grid, dim3(kPartWaves * kWave), 0, stream, part, n_split, n_tokens,
+                       n_expert, k, normalize ? 1 : 0, ids, weights);
+  else if (n_expert <= 128)
+    hipLaunchKernelGGL(router_part_topk_kernel<8>, grid, dim3(kPartWaves * kWave), 0, stream, part, n_split, n_tokens,
+                       n_expert, k, normalize ? 1 : 0, ids, weights);
+  else
+    hipLaunchKernelGGL(router_part_topk_kernel<16>, grid, dim3(kPartWaves * kWave), 0, stream, part, n_split,
+                       n_tokens, n_expert, k, normalize ? 1 : 0, ids, weights);
+  return hipGetLastError();
+}
+
+size_t split_bytes(int n_tokens, int n_embd, int n_expert) {
+  return static_cast<size_t>(router_decode_splits(n_embd)) * n_tokens * n_expert * sizeof(float);
+}
+
+}  // namespace
+
 size_t router_prefill_scratch_bytes(int n_tokens, int n_embd, int n_expert, int k, int dtype) {
+  if (dtype == DT_F32)
+    return n_tokens > kDecodeMaxTokens && f32_split_ok(n_tokens, n_embd, n_expert, k)
+               ? split_bytes(n_tokens, n_embd, n_expert)
+               : 0;
   if (dtype != DT_BF16 || n_tokens <= kDecodeMaxTokens || n_embd % kTileCols || n_expert <= 32 ||
       n_expert > kMfmaMaxExpert || k <= 0 || k > 16 || k > n_expert)
     return 0;
@@ -688,6 +873,15 @@ hipError_t launch_router_prefill(const void* x, const void* wr, int n_tokens, in
   if (!part || router_prefill_scratch_bytes(n_tokens, n_embd, n_expert, k, dtype) == 0 ||
       reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(wr) % 16)
     return hipErrorNotSupported;
+  if (dtype == DT_F32) {
+    const int n_split = router_decode_splits(n_embd);
+    hipLaunchKernelGGL(router_split_logits_f32_kernel, dim3((n_tokens + 15) / 16, (n_expert + 15) / 16, n_split),
+                       dim3(kSplitWaves * kWave), 0, stream, static_cast<const float*>(x),
+                       static_cast<const float*>(wr), n_tokens, n_embd, n_expert, part);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    return launch_part_topk(part, n_split, n_tokens, n_expert, k, normalize, ids, weights, stream);
+  }
   const PrefillSplit ps = prefill_split(n_tokens, n_embd);
   const bf16_t* xb = static_cast<const bf16_t*>(x);
   const bf16_t* wb = static_cast<const bf16_t*>(wr);
@@ -699,22 +893,18 @@ hipError_t launch_router_prefill(const void* x, const void* wr, int n_tokens, in
                              weights, part, stream);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const dim3 grid((n_tokens + 4 * kPartWaves - 1) / (4 * kPartWaves));
-  if (n_expert <= 64)
-    hipLaunchKernelGGL(router_part_topk_kernel<4>, grid, dim3(kPartWaves * kWave), 0, stream, part, ps.n_split,
-                       n_tokens, n_expert, k, normalize ? 1 : 0, ids, weights);
-  else
-    hipLaunchKernelGGL(router_part_topk_kernel<8>, grid, dim3(kPartWaves * kWave), 0, stream, part, ps.n_split,
-                       n_tokens, n_expert, k, normalize ? 1 : 0, ids, weights);
-  return hipGetLastError();
+  return launch_part_topk(part, ps.n_split, n_tokens, n_expert, k, normalize, ids, weights, stream);
 }
 
 size_t router_decode_scratch_bytes(int n_tokens, int n_embd, int n_expert, int k, int dtype) {
+  if (dtype == DT_F32)
+    return n_tokens <= kDecodeMaxTokens && f32_split_ok(n_tokens, n_embd, n_expert, k)
+               ? split_bytes(n_tokens, n_embd, n_expert)
+               : 0;
   if (dtype != DT_BF16 || n_tokens <= 0 || n_tokens > kDecodeMaxTokens || n_embd % 32 || n_expert <= 0 ||
       n_expert > 256 || k <= 0 || k > 16 || k > n_expert)
     return 0;
-  const int n_split = (n_embd + kSplitCols - 1) / kSplitCols;
-  return static_cast<size_t>(n_split) * n_tokens * n_expert * sizeof(float);
+  return split_bytes(n_tokens, n_embd, n_expert);
 }
 
 int router_decode_splits(int n_embd) { return (n_embd + kSplitCols - 1) / kSplitCols; }
@@ -725,9 +915,14 @@ hipError_t launch_router_split_logits(const void* x, const void* wr, int n_token
       reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(wr) % 16)
     return hipErrorNotSupported;
   const int n_split = router_decode_splits(n_embd);
-  hipLaunchKernelGGL(router_split_logits_kernel, dim3((n_tokens + 15) / 16, (n_expert + 15) / 16, n_split),
-                     dim3(kSplitWaves * kWave), 0, stream, static_cast<const bf16_t*>(x),
-                     static_cast<const bf16_t*>(wr), n_tokens, n_embd, n_expert, part);
+  const dim3 grid((n_tokens + 15) / 16, (n_expert + 15) / 16, n_split);
+  if (dtype == DT_F32)
+    hipLaunchKernelGGL(router_split_logits_f32_kernel, grid, dim3(kSplitWaves * kWave), 0, stream,
+                       static_cast<const float*>(x), static_cast<const float*>(wr), n_tokens, n_embd, n_expert, part);
+  else
+    hipLaunchKernelGGL(router_split_logits_kernel, grid, dim3(kSplitWaves * kWave), 0, stream,
+                       static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(wr), n_tokens, n_embd, n_expert,
+                       part);
   *n_split_out = n_split;
   return hipGetLastError();
 }
@@ -747,14 +942,7 @@ hipError_t launch_router_decode(const void* x, const void* wr, int n_tokens, int
     // follows as its own launch.  Measured (whole block calls, cold): C3
     // T=64 123.0 -> 119.4 us; at T=16 the fused kernel is ahead (77.3 against
     // 78.8 us), its 4 waves one per SIMD.
-    const dim3 grid((n_tokens + 4 * kPartWaves - 1) / (4 * kPartWaves));
-    if (nv <= 8)
-      hipLaunchKernelGGL(router_part_topk_kernel<8>, grid, dim3(kPartWaves * kWave), 0, stream, part, n_split,
-                         n_tokens, n_expert, k, normalize ? 1 : 0, ids, weights);
-    else
-      hipLaunchKernelGGL(router_part_topk_kernel<16>, grid, dim3(kPartWaves * kWave), 0, stream, part, n_split,
-                         n_tokens, n_expert, k, normalize ? 1 : 0, ids, weights);
-    const hipError_t e2 = hipGetLastError();
+    const hipError_t e2 = launch_part_topk(part, n_split, n_tokens, n_expert, k, normalize, ids, weights, stream);
     if (e2 != hipSuccess) return e2;
     return launch_permute(ids, k * n_tokens, n_expert, order, offsets, err_count, nullptr, stream);
   }

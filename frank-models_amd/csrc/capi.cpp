@@ -803,8 +803,7 @@ AttnLayout attn_layout(const AttnShape& a, int64_t max_ctx, int act) {
 // kernel takes the Q/K/V product from 39 to 32 us, at 128 rows from 88 (the
 // unsplit tile kernel) to 38 us and the output projection from 84 to 31 us;
 // at 32 rows streaming is ahead (Q/K/V 27 against 29 us).  The fused
-// epilogues below stream up to 64 rows (the output projection with its bias
-// and residual at 64 rows: 24.7 us, level with the split product + launch).
+// projections below go first, up to gemm_stream_fused_rows rows.
 constexpr int kLinearStreamRows = 32;
 
 // out[B, N] fp32 = x[B, K] @ W for a one-expert packed weight [N, K].  The
@@ -844,13 +843,13 @@ int run_linear(const void* x, int64_t K, const void* packed, const float* scales
   // Decode batches read each weight once in the streaming kernel (see
   // kLinearStreamRows), with up to ~2048 blocks and at least 4 input steps
   // per wave.
-  if (g_path.load(std::memory_order_relaxed) == FMOE_PATH_AUTO && B <= 64 && pe && fused) {
+  if (g_path.load(std::memory_order_relaxed) == FMOE_PATH_AUTO && pe && fused) {
     GroupedGemmArgs f = g;
     f.epi = pe->kind;
     f.pe = *pe;
     f.out = pe->kind == EPI_LINEAR ? pe->out : nullptr;
     f.out_dtype = FMOE_BF16;
-    if (gemm_stream_supported(f)) {
+    if (gemm_stream_supported(f) && B <= gemm_stream_fused_rows(f)) {
       FMOE_HIP(launch_gemm_stream(f, s));
       g_last_path = FMOE_PATH_STREAM;
       *fused = true;
@@ -935,12 +934,10 @@ int run_attention(const AttnShape& a, const AttnWeights& w, const void* input, c
   const bool bias = w.use_bias != 0;
   {
     ScopedTimer t(FMOE_TIMER_QKV, s);
-    // bias + RoPE in the GEMM's epilogue where the streaming kernel takes
-    // it, else over the fp32 (K-split) result.  Fused only up to 16 rows:
-    // the epilogue's double-precision angles run on one wave per block, and
-    // at 64 rows the separate RoPE launch is faster (Q/K/V phase 38.6
-    // against 44.5 us fused at 64 x 1024 positions).  At 16 x 4096 the
-    // fused step is 1.3 us shorter, at 1 x 512 3.5 us (43.0 -> 39.5 us).
+    // bias + RoPE in the GEMM's epilogue where a streaming kernel takes it
+    // (gemm_stream_fused_rows), else over the fp32 (K-split) result.  At 16
+    // x 4096 the fused step is 1.3 us shorter, at 1 x 512 3.5 us (43.0 ->
+    // 39.5 us).
     ProjEpilogue pe;
     pe.kind = EPI_QKV_ROPE;
     pe.bias = bias ? w.bq : nullptr;
@@ -958,7 +955,7 @@ int run_attention(const AttnShape& a, const AttnWeights& w, const void* input, c
     int ns = 1;
     bool fused = false;
     FMOE_TRY(run_linear(input, a.n_embd, w.wqkv, w.wqkv_scales, w.w_dtype, nq + 2 * nkv, qkv, B, act, order,
-                        offsets, s, &ns, act == FMOE_BF16 && B <= 16 ? &pe : nullptr, &fused));
+                        offsets, s, &ns, act == FMOE_BF16 ? &pe : nullptr, &fused));
     if (!fused)
       FMOE_HIP(launch_qkv_rope(qkv, ns, static_cast<int64_t>(B) * (nq + 2 * nkv), bias ? w.bq : nullptr,
                                bias ? w.bk : nullptr, bias ? w.bv : nullptr, positions, B, nq, nkv,

@@ -64,11 +64,18 @@ __device__ __forceinline__ float silu_mul(float g, float u) {
 // rotation's fused multiply-adds are written out so that every kernel that
 // applies it rounds the same way (left to the compiler, the contraction of
 // a * c - b * s may pick either product).
-__device__ __forceinline__ float2 rope_cos_sin(int64_t pos, int i, int D, double freq_base, double freq_scale) {
-  const double freq = freq_scale / pow(freq_base, static_cast<double>(2 * i) / D);
+__device__ __forceinline__ double rope_freq(int i, int D, double freq_base, double freq_scale) {
+  return freq_scale / pow(freq_base, static_cast<double>(2 * i) / D);
+}
+
+__device__ __forceinline__ float2 rope_cos_sin(int64_t pos, double freq) {
   double sn, cs;
   sincos(static_cast<double>(pos) * freq, &sn, &cs);
   return float2{static_cast<float>(cs), static_cast<float>(sn)};
+}
+
+__device__ __forceinline__ float2 rope_cos_sin(int64_t pos, int i, int D, double freq_base, double freq_scale) {
+  return rope_cos_sin(pos, rope_freq(i, D, freq_base, freq_scale));
 }
 
 __device__ __forceinline__ void rope_apply(float x0, float x1, float2 cs, float& y0, float& y1) {

@@ -24,8 +24,9 @@
 //   stream  decode-sized batches: every weight block is read exactly once
 //           straight into MFMA registers (no LDS), 16 assignment rows per
 //           pass, 8 input steps of loads in flight per wave (16 for the
-//           one-tile bf16 gate/up kernel); one-weight projections of at most
-//           16 rows stream through a ring in LDS instead (gemm_stream_lds_kernel).
+//           one-tile bf16 gate/up kernel); one-weight projections stream
+//           through a ring in LDS instead (gemm_stream_lds_kernel up to 16
+//           rows, gemm_proj_kernel up to 128 and with fp8 weights).
 //           For decode batches of at most 4 tokens the gate/up kernel can run
 //           the router's top-k and grouping in its own blocks (RoutePrologue),
 //           one launch fewer.
@@ -705,6 +706,196 @@ __global__ __launch_bounds__(kThreads + kRopeWaves * kWave) void gemm_stream_lds
   }
 }
 
+// ============================================= projections of 17 to 128 rows
+// The same projections for more rows (and with fp8 weights): block = 16 * NB
+// columns against all MT 16-row tiles, its 4 waves splitting the input axis in
+// units of 64 inputs.  Each wave streams its units through a ring of D slots
+// of its own in LDS (global_load_lds, no staging registers, no barrier in the
+// loop): the unit's weight blocks (non-temporal) and its token rows as
+// 128-byte row segments, 8 rows per load, with the 16-byte chunks of a row at
+// chunk ^ ((row >> 1) & 7) so that an operand read of 16 rows hits all 64
+// banks.  Each weight byte is read once; the token rows come from L2 (once
+// per block), so a block takes two column groups where that still leaves
+// every CU a block.
+// The partial sums are added in wave order through LDS, each wave finishing
+// its share of the (row tile, column group) pairs with the fused epilogue.
+// RoPE: the angles of a wave's pairs are computed before its loop, while its
+// first loads are in flight.
+// Bound: the weights' HBM read plus the token rows' L2 reads (512 KiB per
+// block at 61 rows).  Measured (Mixtral attention, 61 rows, kernel trace):
+// Q/K/V 35 us (a split tile product, its identity grouping and a RoPE
+// launch) -> 20.5 us; output projection 24.4 us (gemm_stream_kernel) -> 13.2
+// us; whole step with 17 / 32 / 64 / 128 rows x 256 positions 57.0 / 62.6 /
+// 85.1 / 112 -> 47.8 / 51.3 / 60.3 / 102 us, and with fp8 weights at 16 / 32 /
+// 64 / 128 rows 46.8 / 62.1 / 77.1 / 105 -> 42.4 / 44.3 / 54.6 / 97.8 us.
+constexpr int kProjMaxRows = 128;
+constexpr int kProjWaves = 4;
+constexpr int kProjThreads = kProjWaves * kWave;
+
+template <int MT, int NB, bool F8>
+struct Proj {
+  static constexpr int kWBytes = NB * (F8 ? 1024 : 2048);  // weight blocks of a unit
+  static constexpr int kSlot = kWBytes + MT * 2048;
+  static constexpr int kLoads = kSlot / 1024;
+  static constexpr int kFit = (152 * 1024) / (kProjWaves * kSlot);
+  static constexpr int D = kFit < 8 ? kFit : 8;
+  static constexpr int kItems = MT * NB;                   // (row tile, column group) pairs
+  static constexpr int kPart = kProjWaves * kItems * 1024; // partial sums, in the drained ring
+  static constexpr int kRing = kProjWaves * D * kSlot;
+  static constexpr int kLds = kRing > kPart ? kRing : kPart;
+  static_assert(D >= 2 && (D - 1) * kLoads <= 63, "two slots, loads within the vmcnt range");
+};
+
+// One wave's loads of unit u into the ring slot at dst.
+template <int MT, int NB, bool F8>
+__device__ __forceinline__ void proj_issue(const unsigned char* const* src, int u, unsigned char* dst) {
+  constexpr int kW = Proj<MT, NB, F8>::kWBytes / 1024, kAll = Proj<MT, NB, F8>::kLoads;
+  // plain variables: the builtin's operands must not depend on the template
+  const int64_t w_ofs = static_cast<int64_t>(u) * (F8 ? 1024 : 2048), t_ofs = static_cast<int64_t>(u) * 128;
+#pragma unroll
+  for (int b = 0; b < kW; ++b)
+    __builtin_amdgcn_global_load_lds(src[b] + w_ofs, dst + b * 1024, 16, 0, kNonTemporal);
+#pragma unroll
+  for (int j = kW; j < kAll; ++j) __builtin_amdgcn_global_load_lds(src[j] + t_ofs, dst + j * 1024, 16, 0, 0);
+}
+
+template <int EPI, int MT, int NB, bool F8>
+__global__ __launch_bounds__(kProjThreads) void gemm_proj_kernel(GroupedGemmArgs g) {
+  static_assert(EPI == EPI_LINEAR || EPI == EPI_QKV_ROPE, "fused one-weight projection epilogues");
+  using P = Proj<MT, NB, F8>;
+  constexpr int D = P::D, kSlot = P::kSlot, kLoads = P::kLoads, kWBytes = P::kWBytes;
+  constexpr int kPerWave = (P::kItems + kProjWaves - 1) / kProjWaves;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int count = g.n_assign;
+  const int64_t N = g.N;
+  const int64_t col0 = static_cast<int64_t>(blockIdx.x) * (16 * NB);
+  const int units = static_cast<int>(g.K / 64);
+  const int u0 = wave * units / kProjWaves;
+  const int n = (wave + 1) * units / kProjWaves - u0;
+  const ProjEpilogue& pe = g.pe;
+
+  // positions of the rows this wave finishes (row tile (wave + 4 i) / NB)
+  int64_t pos[kPerWave];
+  if (EPI == EPI_QKV_ROPE) {
+#pragma unroll
+    for (int i = 0; i < kPerWave; ++i) {
+      const int r = (wave + kProjWaves * i) / NB * 16 + (lane & 15);
+      pos[i] = pe.positions[r < count ? r : 0];
+    }
+  }
+
+  // Sources of one unit: weight block b of the unit (bf16: column group b /
+  // 2, 32-input step b % 2; fp8: column group b), then rows 8 j .. 8 j + 7.
+  constexpr int kWB = kWBytes / 1024;
+  const unsigned char* src[kLoads];
+#pragma unroll
+  for (int b = 0; b < kWB; ++b) {
+    const int64_t cg = static_cast<int64_t>(blockIdx.x) * NB + (F8 ? b : b / 2);
+    src[b] = static_cast<const unsigned char*>(g.w0) +
+             (cg * (F8 ? units : 2 * units) + (F8 ? u0 : 2 * u0 + (b & 1))) * 1024 + lane * 16;
+  }
+#pragma unroll
+  for (int j = 0; j < 2 * MT; ++j) {
+    const int r = 8 * j + (lane >> 3);
+    src[kWB + j] = reinterpret_cast<const unsigned char*>(static_cast<const bf16_t*>(g.a) +
+                                                          static_cast<int64_t>(r < count ? r : 0) * g.lda +
+                                                          static_cast<int64_t>(u0) * 64) +
+                   ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+  }
+  unsigned char* ring = lds + wave * (D * kSlot);
+  for (int u = 0; u < D && u < n; ++u) proj_issue<MT, NB, F8>(src, u, ring + u * kSlot);
+
+  // A wave's pairs all lie in column group wave % NB (NB divides the wave
+  // count), so its lanes need two frequencies each.  v columns take none.
+  static_assert(kProjWaves % NB == 0, "one column group per wave");
+  float2 cs[kPerWave][2];
+  const int64_t rc = col0 + wave % NB * 16 + 4 * (lane >> 4);
+  if (EPI == EPI_QKV_ROPE && rc < static_cast<int64_t>(pe.nq) + pe.nkv) {
+    const int i0 = static_cast<int>((rc < pe.nq ? rc : rc - pe.nq) % pe.head_dim) / 2;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const double freq = rope_freq(i0 + h, pe.head_dim, pe.freq_base, pe.freq_scale);
+#pragma unroll
+      for (int i = 0; i < kPerWave; ++i) cs[i][h] = rope_cos_sin(pos[i], freq);
+    }
+  }
+
+  f32x4_t acc[MT][NB];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[mt][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  int slot = 0;
+  const int r16 = lane & 15, q = lane >> 4;
+  for (int u = 0; u < n; ++u) {
+    // unit u has arrived once at most the loads of the D - 1 younger units
+    // are in flight (loads complete in order); near the end, wait for all
+    if (u + D <= n)
+      __builtin_amdgcn_s_waitcnt(wait_vm((D - 1) * kLoads, false));
+    else
+      __builtin_amdgcn_s_waitcnt(wait_vm(0, false));
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    const unsigned char* sl = ring + slot * kSlot;
+    u32x4_t w[NB][2];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      if (F8) {
+        f8x16_to_bf16(*reinterpret_cast<const u32x4_t*>(sl + nb * 1024 + lane * 16), w[nb][0], w[nb][1]);
+      } else {
+        w[nb][0] = *reinterpret_cast<const u32x4_t*>(sl + nb * 2048 + lane * 16);
+        w[nb][1] = *reinterpret_cast<const u32x4_t*>(sl + nb * 2048 + 1024 + lane * 16);
+      }
+    }
+    u32x4_t t[MT][2];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        t[mt][h] = *reinterpret_cast<const u32x4_t*>(sl + kWBytes + mt * 2048 + r16 * 128 +
+                                                     (((4 * h + q) ^ ((r16 >> 1) & 7)) << 4));
+    __builtin_amdgcn_sched_barrier(0);  // every read in flight before the first MFMA
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) acc[mt][nb] = mfma16(w[nb][h], t[mt][h], acc[mt][nb]);
+    // the slot is refilled only after its reads have returned
+    __builtin_amdgcn_s_waitcnt(wait_vm(63, true));
+    __builtin_amdgcn_sched_barrier(0);
+    if (u + D < n) proj_issue<MT, NB, F8>(src, u + D, ring + slot * kSlot);
+    slot = slot + 1 == D ? 0 : slot + 1;
+  }
+
+  f32x4_t* part = reinterpret_cast<f32x4_t*>(lds);
+  __syncthreads();
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) part[(wave * P::kItems + mt * NB + nb) * kWave + lane] = acc[mt][nb];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kPerWave; ++i) {
+    const int item = wave + kProjWaves * i;
+    if (item >= P::kItems) break;
+    f32x4_t v = part[item * kWave + lane];
+#pragma unroll
+    for (int w = 1; w < kProjWaves; ++w) v += part[(w * P::kItems + item) * kWave + lane];
+    const int r = item / NB * 16 + r16;
+    const int64_t c = col0 + (item % NB) * 16 + 4 * q;
+    if (r >= count || c >= N) continue;
+    if (F8) {
+      const float4 sc = *reinterpret_cast<const float4*>(g.s0 + c);
+      v = f32x4_t{v[0] * sc.x, v[1] * sc.y, v[2] * sc.z, v[3] * sc.w};
+    }
+    store4_proj<EPI, EPI == EPI_QKV_ROPE>(g, r, c, v[0], v[1], v[2], v[3], cs[i][0], cs[i][1]);
+  }
+}
+
 // ============================================================ down + combine
 // Decode batches whose n_assign = n_tokens * k assignments fit one 16-row
 // MFMA tile (n_assign <= 16): the down projection and the slot-ordered
@@ -934,8 +1125,8 @@ void launch_stream_tiles(const GroupedGemmArgs& g, hipStream_t s, dim3 grid, int
     hipLaunchKernelGGL((gemm_stream_kernel<EPI_SWIGLU, 2, F8, TILES>), grid, dim3(kThreads), 0, s, g, col_tiles);
   else if (g.epi == EPI_LINEAR)
     hipLaunchKernelGGL((gemm_stream_kernel<EPI_LINEAR, 1, F8, TILES>), grid, dim3(kThreads), 0, s, g, col_tiles);
-  else if (g.epi == EPI_QKV_ROPE)
-    hipLaunchKernelGGL((gemm_stream_kernel<EPI_QKV_ROPE, 1, F8, TILES>), grid, dim3(kThreads), 0, s, g, col_tiles);
+  else if (g.epi == EPI_QKV_ROPE)  // up to 16 rows (gemm_stream_fused_rows)
+    hipLaunchKernelGGL((gemm_stream_kernel<EPI_QKV_ROPE, 1, F8, 1>), grid, dim3(kThreads), 0, s, g, col_tiles);
   else if (g.epi == EPI_SCATTER_WEIGHTED)
     hipLaunchKernelGGL((gemm_stream_kernel<EPI_SCATTER_WEIGHTED, 1, F8, TILES>), grid, dim3(kThreads), 0, s, g,
                        col_tiles);
@@ -1022,6 +1213,40 @@ hipError_t launch_stream_routed(const GroupedGemmArgs& g, hipStream_t s, int col
   return hipLaunchKernel(k, dim3(blocks), dim3(kThreads), args, 0, s);
 }
 
+template <int EPI, int MT, int NB, bool F8>
+hipError_t launch_proj_n(const GroupedGemmArgs& g, hipStream_t s) {
+  constexpr int lds = Proj<MT, NB, F8>::kLds;
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_proj_kernel<EPI, MT, NB, F8>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  (void)attr;
+  const dim3 grid(static_cast<unsigned>((g.N + 16 * NB - 1) / (16 * NB)));
+  hipLaunchKernelGGL((gemm_proj_kernel<EPI, MT, NB, F8>), grid, dim3(kProjThreads), lds, s, g);
+  return hipGetLastError();
+}
+
+// Two column groups per block above 256 groups: a block then reads its token
+// rows for twice the columns and the grid is one round of one block per CU.
+template <int EPI, int MT, bool F8>
+hipError_t launch_proj_m(const GroupedGemmArgs& g, hipStream_t s) {
+  if (g.N > 16 * 256 && g.N % 32 == 0) {
+    if constexpr (MT <= 4) return launch_proj_n<EPI, MT, 2, F8>(g, s);
+  }
+  return launch_proj_n<EPI, MT, 1, F8>(g, s);
+}
+
+template <int EPI, bool F8>
+hipError_t launch_proj(const GroupedGemmArgs& g, hipStream_t s) {
+  const int mt = (g.n_assign + 15) / 16;
+  if constexpr (F8) {  // bf16 weights take gemm_stream_lds_kernel up to 16 rows
+    if (mt <= 1) return launch_proj_m<EPI, 1, F8>(g, s);
+  }
+  if (mt <= 2) return launch_proj_m<EPI, 2, F8>(g, s);
+  if (mt <= 3) return launch_proj_m<EPI, 3, F8>(g, s);
+  if (mt <= 4) return launch_proj_m<EPI, 4, F8>(g, s);
+  if (mt <= 6) return launch_proj_m<EPI, 6, F8>(g, s);
+  return launch_proj_m<EPI, 8, F8>(g, s);
+}
+
 template <bool F8>
 hipError_t launch_stream_t(const GroupedGemmArgs& g, hipStream_t s) {
   const int col_tiles = static_cast<int>((g.N + kStreamRows - 1) / kStreamRows);
@@ -1054,6 +1279,8 @@ hipError_t launch_stream_t(const GroupedGemmArgs& g, hipStream_t s) {
                          dim3(stream_lds_threads<EPI_QKV_ROPE>()), (stream_lds_bytes<kDepth, EPI_QKV_ROPE>()), s, g);
     return hipGetLastError();
   }
+  if ((g.epi == EPI_LINEAR || g.epi == EPI_QKV_ROPE) && g.K % 64 == 0 && g.n_assign <= kProjMaxRows)
+    return g.epi == EPI_LINEAR ? launch_proj<EPI_LINEAR, F8>(g, s) : launch_proj<EPI_QKV_ROPE, F8>(g, s);
   if (rows <= 16)
     launch_stream_tiles<F8, 1>(g, s, grid, col_tiles);
   else if (rows <= 32)
@@ -1081,6 +1308,15 @@ bool proj_epilogue_ok(const GroupedGemmArgs& g) {
          al8(e.k_out) && al8(e.v_out) && e.nq > 0 && e.nkv > 0 && e.nq % 4 == 0 && e.nkv % 4 == 0 &&
          e.head_dim > 0 && e.head_dim % 4 == 0 && e.nq % e.head_dim == 0 && e.nkv % e.head_dim == 0 &&
          g.N == static_cast<int64_t>(e.nq) + 2 * e.nkv;
+}
+
+// gemm_proj_kernel's range where it runs (its comment has both sides); the
+// register kernel's otherwise: its RoPE epilogue's angles run on one wave per
+// block (Q/K/V at 64 rows 44.5 us against 38.6 with a launch of their own), its
+// output projection streams up to 64 rows (24.7 us, level with the split
+// product + launch).
+int gemm_stream_fused_rows(const GroupedGemmArgs& g) {
+  return g.K % 64 == 0 ? kProjMaxRows : g.epi == EPI_LINEAR ? 64 : 16;
 }
 
 bool gemm_stream_routed_ok(const GroupedGemmArgs& g) {

@@ -271,6 +271,10 @@ hipError_t launch_down_combine_small(const GroupedGemmArgs& d, const void* resid
                                      int n_tokens, int k, hipStream_t stream);
 bool gemm_tiled_supported(const GroupedGemmArgs& g);
 bool gemm_stream_supported(const GroupedGemmArgs& g);
+// Rows up to which a projection should take its fused epilogue (g.epi
+// EPI_LINEAR / EPI_QKV_ROPE, supported): beyond, the split product and a
+// launch for the bias / RoPE are faster.
+int gemm_stream_fused_rows(const GroupedGemmArgs& g);
 // Whether the streaming gate/up GEMM takes g with its routing (g.rp set):
 // the shape qualifies and the grid fits one round of resident blocks.
 bool gemm_stream_routed_ok(const GroupedGemmArgs& g);

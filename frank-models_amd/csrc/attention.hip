@@ -12,14 +12,14 @@
 // place instead of gathering: the zero rows' contribution is exact in closed
 // form (score 0, value 0), so they are counted, not read.
 //
-// Attention is split over the context: one block per (split of kSplitLen
-// positions, KV head, sequence) computes, for the G query heads sharing the
+// Attention is split over the context: one block per (split of positions, KV
+// head, sequence) computes, for the G query heads sharing the
 // KV head, the split's max score, sum of exp and unnormalised output; a
 // combine kernel merges the splits in order with the zero rows and the new
 // token and, in the paged calls, writes the new K/V rows into the pools.
 // Where the streaming GEMM does not apply its own epilogue (fp32
-// activations, more than 16 rows for Q/K/V), the separate bias + RoPE and
-// bias + cast kernels here finish the projections.
+// activations, more rows than gemm_stream_fused_rows), the separate bias +
+// RoPE and bias + cast kernels here finish the projections.
 #include "common.h"
 #include "launch.h"
 
@@ -212,6 +212,7 @@ struct AttnArgs {
   int block_size;
   int n_head, n_head_kv;
   int n_split;
+  int split_len;          // positions per split
   float scale;
   float* part;            // [B, n_head, n_split, D + 2]: o[D], m, l
 };
@@ -221,8 +222,10 @@ constexpr int kAttnThreads = 256;  // one thread per position of a split (rows[]
 static_assert(kAttnThreads == kSplitLen, "the rows[] fill gives each thread one position");
 constexpr int kAttnWaves = kAttnThreads / kWave;
 
-// Block (split s, KV head, sequence b); wave w owns the split's positions
-// [64 w, 64 w + 64) in both phases, so a wave's memory traffic is two
+// fp32 pools, head_dim 16 and 32, and bf16 pools that are not 16-byte aligned
+// (attn_ring_kernel below takes the others).
+// Block (split s of kSplitLen positions, KV head, sequence b); wave w owns the
+// split's positions [64 w, 64 w + 64) in both phases, so a wave's memory traffic is two
 // rounds of independent loads: all of its K rows, then (issued before the
 // block-wide softmax, so that their latency overlaps it) all of its V rows.
 // Scores: LP lanes per position, each lane holding DL = D/LP dimensions in
@@ -247,7 +250,6 @@ __global__ __launch_bounds__(kAttnThreads) void attn_split_kernel(AttnArgs a) {
   constexpr int NV = kQ / PP;                             // V load instructions per wave
   constexpr int VR = NV < 16 ? NV : 16;                   // per round
   static_assert(kSteps % SR == 0 && NV % VR == 0, "rounds must tile the wave's positions");
-  constexpr bool kMfmaScores = sizeof(T) == 2 && (D == 64 || D == 128) && G <= 8 && kQ % 8 == 0;
   __shared__ float sc[G][kSplitLen];
   __shared__ int rows[kSplitLen];
   __shared__ float red[kAttnWaves][G][D];
@@ -259,13 +261,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_split_kernel(AttnArgs a) {
   const int j0 = s * kSplitLen;
   const int len = min(kSplitLen, n_b - j0);  // block-uniform; <= 0: no cached position here
   float* part = a.part + (static_cast<int64_t>(b) * a.n_head + kvh * G) * a.n_split * (D + 2);
-  if (len <= 0) {
-    for (int i = tid; i < G * (D + 2); i += kAttnThreads) {
-      const int g = i / (D + 2), k = i - g * (D + 2);
-      part[(static_cast<int64_t>(g) * a.n_split + s) * (D + 2) + k] = k == D ? -INFINITY : 0.f;
-    }
-    return;
-  }
+  if (len <= 0) return;  // the combine reads only the splits with positions
   const int64_t row_elems = static_cast<int64_t>(a.n_head_kv) * D;
   {
     const int t = tid;  // kAttnThreads == kSplitLen: one position per thread
@@ -281,62 +277,6 @@ __global__ __launch_bounds__(kAttnThreads) void attn_split_kernel(AttnArgs a) {
   const T* kp = static_cast<const T*>(a.k_pool) + static_cast<int64_t>(kvh) * D;
   const T* vp = static_cast<const T*>(a.v_pool) + static_cast<int64_t>(kvh) * D;
   const int tw = wave * kQ;  // this wave's first position
-  if constexpr (kMfmaScores) {
-    // ---- scores on the matrix cores (v_mfma_f32_16x16x32_bf16), 8
-    // positions per tile.  A row i = 2p + s holds half s of position p's K
-    // row, B column j = 2h + s' half s' of query head h (heads >= G zero):
-    // at step ks, lane group kg (lane >> 4) of row / column parity s takes
-    // the 8 dimensions of chunk 8 ks + 4 s + kg, so the 8 lanes of a
-    // position read 128 contiguous bytes per load.  score(p, h) =
-    // D[2p][2h] + D[2p+1][2h+1]; the cross terms (s != s') are unused.  q is
-    // split into bf16 high and low parts (two MFMAs per step): the products
-    // carry q * scale to about 16 significant bits, K is exact in bf16 and
-    // the sums are fp32.
-    constexpr int NKS = D / 64, PT = kQ / 8;
-    const int kg = lane >> 4, par = lane & 1, hh = (lane & 15) >> 1;
-    u32x4_t qh[NKS], ql[NKS];
-    {
-      const float* qg = a.q + (static_cast<int64_t>(b) * a.n_head + kvh * G + (hh < G ? hh : 0)) * D;
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int d = (ks * 8 + par * 4 + kg) * 8 + 2 * e;
-          const float x0 = hh < G ? qg[d] * a.scale : 0.f;
-          const float x1 = hh < G ? qg[d + 1] * a.scale : 0.f;
-          const uint32_t h = pack_bf16x2(x0, x1);
-          qh[ks][e] = h;
-          ql[ks][e] = pack_bf16x2(x0 - __uint_as_float(h << 16), x1 - __uint_as_float(h & 0xFFFF0000u));
-        }
-    }
-    __syncthreads();  // rows[]
-    u32x4_t kr[PT][NKS];
-#pragma unroll
-    for (int pt = 0; pt < PT; ++pt) {
-      const int r = rows[tw + pt * 8 + hh];
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks)
-        kr[pt][ks] = r >= 0 ? *reinterpret_cast<const u32x4_t*>(kp + r * row_elems + (ks * 8 + par * 4 + kg) * 8)
-                            : u32x4_t{0u, 0u, 0u, 0u};
-    }
-#pragma unroll
-    for (int pt = 0; pt < PT; ++pt) {
-      f32x4_t c{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) {
-        c = attn_mfma16(kr[pt][ks], qh[ks], c);
-        c = attn_mfma16(kr[pt][ks], ql[ks], c);
-      }
-      // lane (kg, column 2h + s'): c[r] = D[4 kg + r][2h + s'], rows 4 kg + r
-      // = position 2 kg + (r >> 1), half r & 1
-      const float odd1 = __shfl_xor(c[1], 1, kWave), odd3 = __shfl_xor(c[3], 1, kWave);
-      if (par == 0 && hh < G) {
-        const int t = tw + pt * 8 + 2 * kg;
-        sc[hh][t] = rows[t] == -2 ? -INFINITY : c[0] + odd1;  // a zero row scores 0
-        sc[hh][t + 1] = rows[t + 1] == -2 ? -INFINITY : c[2] + odd3;
-      }
-    }
-  } else {
   const int pi = lane / LP, sub = lane % LP;
   float q[G][DL];
 #pragma unroll
@@ -397,7 +337,6 @@ __global__ __launch_bounds__(kAttnThreads) void attn_split_kernel(AttnArgs a) {
         if (sub == g) sc[g][t] = rr[u] == -2 ? -INFINITY : acc;  // a zero row scores 0
       }
     }
-  }
   }
 
   // ---- V rows of this wave, first round issued before the softmax
@@ -491,6 +430,331 @@ __global__ __launch_bounds__(kAttnThreads) void attn_split_kernel(AttnArgs a) {
   }
 }
 
+// bf16 pools with head_dim 64 or 128 (16-byte aligned pools): the same block
+// (split, KV head, sequence) and partial results, with no block barrier
+// between its loads.  A block's positions (split_len of them: 256, 512 or
+// 1024) go to its waves in chunks of 64, chunk i to wave i % 4.  A chunk is
+// four 16-position tiles of K, then four of V, which pass through a ring of
+// kSlots tiles of the wave's own in LDS (global_load_lds): a slot is refilled
+// as soon as its tile has been used, so loads stay in flight through the
+// score, softmax and P.V arithmetic and across the chunks, and nothing keeps
+// the waves of a CU in step.
+// Bound: the K and V rows' HBM read.  Measured (8 KV heads x 128, 32 query
+// heads, kernel trace; before: every load of a phase in registers, two block
+// barriers around the softmax): 16 sequences x 4096 positions 61.4 -> 50.7 us
+// (5.3 TB/s), 61 x about 750 positions 52.3 -> 42.2 us.
+// Scores: v_mfma_f32_16x16x32_bf16, A = 16 positions x 32 dimensions of K, B
+// column h = query head h (G <= 8), column 8 + h its remainder: q * scale as
+// bf16 high and low parts, about 16 significant bits; K is exact in bf16 and
+// the sums are fp32.  K tiles sit in LDS with 16-byte chunk c of row r at
+// c ^ (r & 15) (head_dim 64: c ^ ((r >> 1) & 7)), so an operand read of 16
+// rows hits all 64 banks.  Softmax per wave in fp32, with a running maximum
+// over its chunks.  P.V: 16 bytes of a row per lane in the loads' own lane
+// order, fp32; load i of a V tile holds positions kLoads * (lane's row) + i,
+// so a lane's probabilities of a tile are neighbours in LDS.
+// Rows past the context (-2) and zero rows (-1, table entries outside the
+// pool) load some valid row instead; their scores are replaced and their
+// values zeroed by selects, so what they loaded never enters the result.
+constexpr int kTileRows = 16;
+constexpr int kSlots = 4;
+constexpr int kChunk = 64;      // positions of a wave per round of the ring
+constexpr int kMaxSplitLen = 1024;
+
+template <int D, int G>
+struct Ring {
+  static constexpr int kRowB = D * 2;
+  static constexpr int kRowsPerLoad = 1024 / kRowB;             // 4 or 8
+  static constexpr int kLoads = kTileRows / kRowsPerLoad;       // per tile
+  static constexpr int kTileB = kTileRows * kRowB;
+  static constexpr int kTiles = kChunk / kTileRows;             // of K, and of V, per chunk
+  static constexpr int kWaveB = kSlots * kTileB;
+  static constexpr int kRowIds = kMaxSplitLen / kAttnWaves;     // per wave
+  static constexpr int kP = kChunk * G;                         // probabilities per wave
+  static constexpr int kLds = kAttnWaves * (kWaveB + kRowIds * 4 + kP * 4 + G * 8);
+  // blocks per CU the registers must allow
+  static constexpr int kBlocks = (D == 64 ? 3 : 2) - (G == 8 ? 1 : 0);
+  static_assert(kSlots == kTiles, "K tile i and V tile i share slot i");
+  static_assert(kWaveB >= 2 * G * D * 4, "a wave's two partial outputs fit its ring");
+};
+
+// Non-temporal: a step reads each K and V byte once (with the default policy
+// the kernel takes 55.5 us at 16 x 4096 positions and 44.9 at 61 x 750).
+__device__ __forceinline__ void ring_load(const unsigned char* src, unsigned char* dst) {
+  __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 2);
+}
+
+template <int D, int G>
+__global__ __launch_bounds__(kAttnThreads, (Ring<D, G>::kBlocks)) void attn_ring_kernel(AttnArgs a) {
+  using R = Ring<D, G>;
+  constexpr int kL = R::kLoads, kT = R::kTiles, kChunks = R::kRowB / 16;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+  const int s = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  unsigned char* ring = lds + wave * R::kWaveB;
+  int* rows = reinterpret_cast<int*>(lds + kAttnWaves * R::kWaveB) + wave * R::kRowIds;
+  float* pw = reinterpret_cast<float*>(lds + kAttnWaves * (R::kWaveB + R::kRowIds * 4)) + wave * R::kP;  // [G][64]
+  float* stat = reinterpret_cast<float*>(lds + kAttnWaves * (R::kWaveB + R::kRowIds * 4 + R::kP * 4));  // [waves][G][m, l]
+
+  // Query operand: lane (g = l / 16, column l % 16) holds 8 dimensions at
+  // chunk 4 ks + g of head l % 8, the high part in columns 0-7, the remainder
+  // in 8-15.  Loaded beside the table entries and the context length, and
+  // converted before the first tile load is issued (a wait for it later
+  // would wait for those loads too).
+  const int q4 = lane >> 4, col = lane & 15, head = col & 7;
+  const float* qg = a.q + (static_cast<int64_t>(b) * a.n_head + kvh * G + (head < G ? head : 0)) * D + q4 * 8;
+  f32x4_t qx[D / 32][2];
+#pragma unroll
+  for (int ks = 0; ks < D / 32; ++ks) {
+    qx[ks][0] = *reinterpret_cast<const f32x4_t*>(qg + ks * 32);
+    qx[ks][1] = *reinterpret_cast<const f32x4_t*>(qg + ks * 32 + 4);
+  }
+  // Pool rows of the wave's positions, chunk by chunk.
+  const int j0 = s * a.split_len;
+  const int n_b = min(max(a.ctx_lens[b], 0), a.max_ctx);
+  if (n_b <= j0) return;  // block-uniform; the combine reads only the splits with positions
+  const int len = min(a.split_len, n_b - j0);
+  const int n_all = (len + kChunk - 1) / kChunk;
+  const int n = n_all > wave ? (n_all - wave + kAttnWaves - 1) / kAttnWaves : 0;  // this wave's chunks
+  for (int c = 0; c < n; ++c) {
+    const int t = (c * kAttnWaves + wave) * kChunk + lane;
+    const int j = j0 + t;
+    const int lb = j / a.block_size;
+    int r = -2;  // past the context
+    if (t < len) {
+      const int pb = lb < a.max_blocks ? a.tables[static_cast<int64_t>(b) * a.max_blocks + lb] : -1;
+      r = pb >= 0 && pb < a.n_blocks ? pb * a.block_size + (j - lb * a.block_size) : -1;
+    }
+    rows[c * kChunk + lane] = r;
+  }
+
+  u32x4_t qv[D / 32];
+#pragma unroll
+  for (int ks = 0; ks < D / 32; ++ks)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float y0 = qx[ks][e / 2][2 * (e % 2)] * a.scale, y1 = qx[ks][e / 2][2 * (e % 2) + 1] * a.scale;
+      const uint32_t h = pack_bf16x2(y0, y1);
+      const uint32_t lo = pack_bf16x2(y0 - __uint_as_float(h << 16), y1 - __uint_as_float(h & 0xFFFF0000u));
+      qv[ks][e] = head < G ? (col < 8 ? h : lo) : 0u;
+    }
+#pragma unroll
+  for (int ks = 0; ks < D / 32; ++ks) asm volatile("" : "+v"(qv[ks]));  // converted here
+  float m = -INFINITY, l = 0.f;
+  float acc[G][8];
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[g][e] = 0.f;
+
+  // this lane's row and 16-byte chunk of a load
+  const int lr = lane / kChunks, lc = lane % kChunks;
+  const int64_t row_b = static_cast<int64_t>(a.n_head_kv) * R::kRowB;
+  const unsigned char* kp = static_cast<const unsigned char*>(a.k_pool) + kvh * R::kRowB;
+  const unsigned char* vp = static_cast<const unsigned char*>(a.v_pool) + kvh * R::kRowB + lc * 16;
+  int kc[kL];
+#pragma unroll
+  for (int i = 0; i < kL; ++i) {
+    const int row = i * R::kRowsPerLoad + lr;
+    kc[i] = (lc ^ (D == 128 ? row & 15 : (row >> 1) & 7)) * 16;
+  }
+  uint64_t valid = 0, zero = 0;            // of the chunk whose K tiles are issued last
+  uint64_t valid_now = 0, zero_now = 0;    // of the chunk being computed
+  // Masks of chunk c, and its unusable rows replaced by a usable one.
+  auto chunk_rows = [&](int c) __attribute__((always_inline)) {
+    const int r = rows[c * kChunk + lane];
+    valid = __ballot(r >= 0);
+    zero = __ballot(r == -1);
+    if (valid != ~0ull) {
+      const int first = valid ? __builtin_amdgcn_readlane(r, __builtin_ctzll(valid)) : 0;
+      if (r < 0) rows[c * kChunk + lane] = first;
+    }
+  };
+  if (n > 0) {
+    chunk_rows(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int it = 0; it < kT; ++it)
+#pragma unroll
+      for (int i = 0; i < kL; ++i)
+        ring_load(kp + rows[it * kTileRows + i * R::kRowsPerLoad + lr] * row_b + kc[i],
+                  ring + it * R::kTileB + i * 1024);
+  }
+  for (int c = 0; c < n; ++c) {
+    const bool more = c + 1 < n;
+    const int* rc = rows + c * kChunk;
+    valid_now = valid;
+    zero_now = zero;
+    const bool all = valid_now == ~0ull;
+
+    // ---- scores: lane (g, column): positions 16 tile + 4 g + i.  In flight
+    // behind K tile `it`: the three tiles after it (K, then V)
+    f32x4_t sc[kT];
+#pragma unroll
+    for (int it = 0; it < kT; ++it) {
+      __builtin_amdgcn_s_waitcnt(wait_vm((kSlots - 1) * kL, false));
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("" ::: "memory");
+      const unsigned char* tile = ring + it * R::kTileB + col * R::kRowB;
+      const int sw = D == 128 ? col : col >> 1;
+      u32x4_t kv[D / 32];
+#pragma unroll
+      for (int ks = 0; ks < D / 32; ++ks)
+        kv[ks] = *reinterpret_cast<const u32x4_t*>(tile + (((4 * ks + q4) ^ sw) << 4));
+      int vr[kL];  // the V tile's rows
+#pragma unroll
+      for (int i = 0; i < kL; ++i) vr[i] = rc[it * kTileRows + lr * kL + i];
+      // the slot is refilled after its reads have returned
+      __builtin_amdgcn_s_waitcnt(wait_vm(63, true));
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < kL; ++i) ring_load(vp + vr[i] * row_b, ring + it * R::kTileB + i * 1024);
+      f32x4_t d{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < D / 32; ++ks) d = attn_mfma16(kv[ks], qv[ks], d);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) d[i] += __shfl_xor(d[i], 8, kWave);  // high + low part
+      if (!all) {
+        const uint64_t vm = valid_now >> (4 * q4), zm = zero_now >> (4 * q4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const uint64_t bit = 1ull << (16 * it + i);
+          d[i] = vm & bit ? d[i] : zm & bit ? 0.f : -INFINITY;
+        }
+      }
+      sc[it] = d;
+    }
+    if (more) chunk_rows(c + 1);
+
+    // ---- softmax over the wave's positions so far; every column of a head
+    // agrees
+    const float m_old = m;
+#pragma unroll
+    for (int it = 0; it < kT; ++it)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) m = fmaxf(m, sc[it][i]);
+    m = fmaxf(m, __shfl_xor(m, 16, kWave));
+    m = fmaxf(m, __shfl_xor(m, 32, kWave));
+    float sum = 0.f;
+#pragma unroll
+    for (int it = 0; it < kT; ++it) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        sc[it][i] = __expf(sc[it][i] - m);
+        sum += sc[it][i];
+      }
+      if (col < G) *reinterpret_cast<f32x4_t*>(pw + col * kChunk + 16 * it + 4 * q4) = sc[it];
+    }
+    sum += __shfl_xor(sum, 16, kWave);
+    sum += __shfl_xor(sum, 32, kWave);
+    if (c > 0) {
+      const float f = __expf(m_old - m);
+      l = fmaf(l, f, sum);
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const float fg = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), g));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[g][e] *= fg;
+      }
+    } else {
+      l = sum;
+    }
+
+    // ---- P.V.  In flight behind V tile `it`: the V tiles after it and the
+    // next chunk's K tiles
+#pragma unroll
+    for (int it = 0; it < kT; ++it) {
+      if (more || it == 0)
+        __builtin_amdgcn_s_waitcnt(wait_vm((kSlots - 1) * kL, false));
+      else if (it == 1)
+        __builtin_amdgcn_s_waitcnt(wait_vm(2 * kL, false));
+      else if (it == 2)
+        __builtin_amdgcn_s_waitcnt(wait_vm(kL, false));
+      else
+        __builtin_amdgcn_s_waitcnt(wait_vm(0, false));
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("" ::: "memory");
+      const unsigned char* tile = ring + it * R::kTileB + lane * 16;
+      u32x4_t v[kL];
+      float p[G][kL];
+#pragma unroll
+      for (int i = 0; i < kL; ++i) v[i] = *reinterpret_cast<const u32x4_t*>(tile + i * 1024);
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int i = 0; i < kL; ++i) p[g][i] = pw[g * kChunk + it * kTileRows + lr * kL + i];
+      int kr[kL];  // the next chunk's K tile rows
+#pragma unroll
+      for (int i = 0; i < kL; ++i)
+        kr[i] = more ? rc[kChunk + it * kTileRows + i * R::kRowsPerLoad + lr] : 0;
+      __builtin_amdgcn_s_waitcnt(wait_vm(63, true));
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) {
+#pragma unroll
+        for (int i = 0; i < kL; ++i) ring_load(kp + kr[i] * row_b + kc[i], ring + it * R::kTileB + i * 1024);
+      }
+      if (!all) {
+        const uint64_t vm = valid_now >> (lr * kL);
+#pragma unroll
+        for (int i = 0; i < kL; ++i) v[i] = vm & (1ull << (16 * it + i)) ? v[i] : u32x4_t{0u, 0u, 0u, 0u};
+      }
+#pragma unroll
+      for (int i = 0; i < kL; ++i) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) unpack2(v[i][e], x + 2 * e);
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[g][e] = fmaf(p[g][i], x[e], acc[g][e]);
+      }
+    }
+  }
+
+  // ---- the waves merged in order: each leaves two partial outputs in its
+  // (drained) ring and its statistics
+#pragma unroll
+  for (int o = 2 * kChunks; o < kWave; o <<= 1)
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[g][e] += __shfl_xor(acc[g][e], o, kWave);
+  if (lane < 2 * kChunks) {
+    float* dst = reinterpret_cast<float*>(ring) + (lane / kChunks) * G * D + (lane % kChunks) * 8;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      *reinterpret_cast<f32x4_t*>(dst + g * D) = f32x4_t{acc[g][0], acc[g][1], acc[g][2], acc[g][3]};
+      *reinterpret_cast<f32x4_t*>(dst + g * D + 4) = f32x4_t{acc[g][4], acc[g][5], acc[g][6], acc[g][7]};
+    }
+  }
+  if (lane < G) {
+    stat[(wave * G + lane) * 2] = m;
+    stat[(wave * G + lane) * 2 + 1] = l;
+  }
+  __syncthreads();
+  float* part = a.part + (static_cast<int64_t>(b) * a.n_head + kvh * G) * a.n_split * (D + 2);
+  for (int i = tid; i < G * D; i += kAttnThreads) {
+    const int g = i / D, d = i - g * D;
+    float M = stat[g * 2];
+#pragma unroll
+    for (int w = 1; w < kAttnWaves; ++w) M = fmaxf(M, stat[(w * G + g) * 2]);
+    float o = 0.f, L = 0.f;
+#pragma unroll
+    for (int w = 0; w < kAttnWaves; ++w) {
+      const float* src = reinterpret_cast<const float*>(lds + w * R::kWaveB);
+      const float f = __expf(stat[(w * G + g) * 2] - M);  // 0 for a wave without positions
+      o = fmaf(f, src[i] + src[G * D + i], o);
+      L = fmaf(f, stat[(w * G + g) * 2 + 1], L);
+    }
+    float* pg = part + (static_cast<int64_t>(g) * a.n_split + s) * (D + 2);
+    pg[d] = o;
+    if (d == 0) {
+      pg[D] = M;
+      pg[D + 1] = L;
+    }
+  }
+}
+
 // One block per (query head, sequence) merges the context splits with the
 // zero rows of the gather (max_ctx - min(ctx_len, max_ctx) keys of score 0
 // and value 0) and the new token, whose K/V (RoPE applied) are k_new/v_new.
@@ -523,7 +787,7 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(AttnArgs 
   const int kvh = h / (a.n_head / a.n_head_kv);
   const int n_b = min(max(a.ctx_lens[b], 0), a.max_ctx);
   const int n_zero = a.max_ctx - n_b;
-  const int n_used = (n_b + kSplitLen - 1) / kSplitLen;
+  const int n_used = (n_b + a.split_len - 1) / a.split_len;
   const float* qh = a.q + (static_cast<int64_t>(b) * a.n_head + h) * D;
   const int64_t kv0 = (static_cast<int64_t>(b) * a.n_head_kv + kvh) * D;
   const float* part = a.part + (static_cast<int64_t>(b) * a.n_head + h) * a.n_split * (D + 2);
@@ -589,12 +853,42 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(AttnArgs 
   if (tid < D) store_act(out, act, (static_cast<int64_t>(b) * a.n_head + h) * D + tid, o);
 }
 
-// Lanes per position in the score phase.  For head_dim 128 (bf16, 4 query
-// heads per KV head) 8 lanes beat 16 (61.5 against 77.9 us at 16 x 4096
-// positions, 72.5 us with 16 lanes forced to 4 waves per SIMD), although
-// 16 lanes halve the query registers.
+// Lanes per position in the score phase: 8 beat 16 at head_dim 128 (measured
+// on bf16 pools, 4 query heads per KV head: 61.5 against 77.9 us at 16 x 4096
+// positions), although 16 lanes halve the query registers.
 constexpr int kLanesPerPos64 = 8;
 constexpr int kLanesPerPos128 = 8;
+
+// Positions per split: the most that still gives the GPU two blocks per CU.
+// Longer splits spend fewer prologues and merges (whole step at 16 x 4096
+// positions: 94.3 us with 256, 92.7 with 512, 91.4 with 1024; 128 x 380: 126,
+// 122, 122).
+int ring_split_len(int max_ctx, int64_t heads) {
+  int len = kMaxSplitLen;
+  while (len > kSplitLen && heads * ((max_ctx + len - 1) / len) < 512) len /= 2;
+  return len;
+}
+
+template <int D, int G>
+void launch_ring_n(const AttnArgs& a, int B, hipStream_t s) {
+  constexpr int lds = Ring<D, G>::kLds;
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(attn_ring_kernel<D, G>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  (void)attr;
+  hipLaunchKernelGGL((attn_ring_kernel<D, G>), dim3(a.n_split, a.n_head_kv, B), dim3(kAttnThreads), lds, s, a);
+}
+
+template <int D>
+hipError_t launch_ring(const AttnArgs& a, int G, int B, hipStream_t s) {
+  switch (G) {
+    case 1: launch_ring_n<D, 1>(a, B, s); break;
+    case 2: launch_ring_n<D, 2>(a, B, s); break;
+    case 4: launch_ring_n<D, 4>(a, B, s); break;
+    case 8: launch_ring_n<D, 8>(a, B, s); break;
+    default: return hipErrorNotSupported;
+  }
+  return hipGetLastError();
+}
 
 template <typename T, int D, int LP>
 hipError_t launch_split_g(const AttnArgs& a, int G, int B, hipStream_t s) {
@@ -651,13 +945,18 @@ hipError_t launch_attn_decode(const float* q_rot, const void* k_pool, const void
   a.block_size = block_size;
   a.n_head = n_head;
   a.n_head_kv = n_head_kv;
-  a.n_split = attn_decode_splits(max_ctx);
   a.scale = scale;
   a.part = part;
   const int G = n_head / n_head_kv;
+  const bool ring = dtype == DT_BF16 && (head_dim == 64 || head_dim == 128) &&
+                    reinterpret_cast<uintptr_t>(k_pool) % 16 == 0 && reinterpret_cast<uintptr_t>(v_pool) % 16 == 0;
+  a.split_len = ring ? ring_split_len(max_ctx, static_cast<int64_t>(batch) * n_head_kv) : kSplitLen;
+  a.n_split = (max_ctx + a.split_len - 1) / a.split_len;  // at most attn_decode_splits(max_ctx)
   if (a.n_split > 0) {
-    const hipError_t e = dtype == DT_F32 ? launch_split_d<float>(a, head_dim, G, batch, s)
-                                         : launch_split_d<bf16_t>(a, head_dim, G, batch, s);
+    const hipError_t e = ring && head_dim == 64 ? launch_ring<64>(a, G, batch, s)
+                         : ring                 ? launch_ring<128>(a, G, batch, s)
+                         : dtype == DT_F32      ? launch_split_d<float>(a, head_dim, G, batch, s)
+                                                : launch_split_d<bf16_t>(a, head_dim, G, batch, s);
     if (e != hipSuccess) return e;
   }
   hipLaunchKernelGGL(attn_combine_kernel, dim3(n_head + (scatter ? 2 : 0), batch), dim3(kCombineThreads), 0, s, a,

@@ -480,7 +480,7 @@ struct Ring {
 // Non-temporal: a step reads each K and V byte once (with the default policy
 // the kernel takes 55.5 us at 16 x 4096 positions and 44.9 at 61 x 750).
 __device__ __forceinline__ void ring_load(const unsigned char* src, unsigned char* dst) {
-  __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 2);
+  __builtin_amdgcn_global_load_lds(src, dst, 16, 0, kNonTemporal);
 }
 
 template <int D, int G>

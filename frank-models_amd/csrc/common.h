@@ -19,6 +19,10 @@ typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_t;
 
 constexpr int kWave = 64;
 
+// Cache policy of a load (the builtins' aux operand) whose bytes no other
+// block of the launch reads: it does not push shared data out of L2.
+constexpr int kNonTemporal = 2;
+
 // ---------------------------------------------------------------- numbers
 __device__ __forceinline__ float bf16_to_f32(bf16_t v) {
   return __uint_as_float(static_cast<uint32_t>(v) << 16);

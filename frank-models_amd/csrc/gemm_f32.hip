@@ -12,7 +12,7 @@
 // pair per 16 inputs with no load in flight across them.  Measured
 // (DeepSeek-V2-Lite in fp32, 64 experts x 2048 x 1408, top-6): 500 tokens
 // gate/up 1607 -> 405-440 us (86 TFLOP/s, 3.6 TB/s) and down 1059 -> 202-224
-// us; 64 tokens gate/up 262 us (5.6 TB/s of weights).
+// us; 64 tokens, whole block, 378 us (5.9 TB/s of weights).
 //
 // Block: 256 threads, a tile of BM assignment rows x 32 * WN weight rows,
 // stages of KS inputs through a ring in LDS filled by global_load_lds (16
@@ -118,7 +118,7 @@ __device__ __forceinline__ bool find_block(const GroupedGemmArgs& g, int bm, int
 }
 
 // One wave's loads of stage st into its ring buffer.
-template <int WN, int BM, int LA>
+template <int WN, int BM, int LA, bool NT>
 __device__ __forceinline__ void issue_stage(const float* const* a_src, const float* const* b_src, int st,
                                             unsigned char* lds, int wave) {
   using C = Cfg<WN, BM>;
@@ -129,13 +129,18 @@ __device__ __forceinline__ void issue_stage(const float* const* a_src, const flo
 #pragma unroll
   for (int i = 0; i < LA; ++i) __builtin_amdgcn_global_load_lds(a_src[i] + ofs, a_dst + i * 4096, 16, 0, 0);
 #pragma unroll
-  for (int i = 0; i < C::kLB; ++i) __builtin_amdgcn_global_load_lds(b_src[i] + ofs, b_dst + i * 4096, 16, 0, 0);
+  for (int i = 0; i < C::kLB; ++i) {
+    if (NT)
+      __builtin_amdgcn_global_load_lds(b_src[i] + ofs, b_dst + i * 4096, 16, 0, kNonTemporal);
+    else
+      __builtin_amdgcn_global_load_lds(b_src[i] + ofs, b_dst + i * 4096, 16, 0, 0);
+  }
 }
 
 // The K loop over stages [0, n_st) for MG 16-row groups.  a_src / b_src:
 // this lane's source of each of its wave's loads at stage 0; load i of the
 // wave covers LDS rows (wave + 4 i) * kRowsPerLoad of the A or weight part.
-template <int WN, int BM, int MG>
+template <int WN, int BM, bool NT, int MG>
 __device__ __forceinline__ void k_loop(const float* const* a_src, const float* const* b_src,
                                        int n_st, unsigned char* lds, f32x4_t (*acc)[BM / 16]) {
   using C = Cfg<WN, BM>;
@@ -152,7 +157,7 @@ __device__ __forceinline__ void k_loop(const float* const* a_src, const float* c
   // Stage st is visible to the block after each wave has waited for its own
   // loads of it and the barrier; the barrier also means every wave has
   // finished stage st - 1, whose buffer stage st + kRing - 1 then refills.
-  for (int st = 0; st < C::kRing - 1 && st < n_st; ++st) issue_stage<WN, BM, kLA>(a_src, b_src, st, lds, wave);
+  for (int st = 0; st < C::kRing - 1 && st < n_st; ++st) issue_stage<WN, BM, kLA, NT>(a_src, b_src, st, lds, wave);
   for (int st = 0; st < n_st; ++st) {
     if (st + C::kRing - 1 <= n_st)
       __builtin_amdgcn_s_waitcnt(wait_vm((C::kRing - 2) * kL, true));
@@ -160,7 +165,7 @@ __device__ __forceinline__ void k_loop(const float* const* a_src, const float* c
       __builtin_amdgcn_s_waitcnt(wait_vm(0, true));
     lds_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    if (st + C::kRing - 1 < n_st) issue_stage<WN, BM, kLA>(a_src, b_src, st + C::kRing - 1, lds, wave);
+    if (st + C::kRing - 1 < n_st) issue_stage<WN, BM, kLA, NT>(a_src, b_src, st + C::kRing - 1, lds, wave);
     const unsigned char* as = lds + (st % C::kRing) * C::kStage;
     const unsigned char* bs = as + C::kABytes;
 #pragma unroll
@@ -184,7 +189,7 @@ __device__ __forceinline__ void k_loop(const float* const* a_src, const float* c
   }
 }
 
-template <int WN, int BM, int EPI>
+template <int WN, int BM, int EPI, bool NT>
 __global__ __launch_bounds__(kThreads, (Cfg<WN, BM>::kBlocks)) void gemm_f32_kernel(GroupedGemmArgs g, int n_col) {
   using C = Cfg<WN, BM>;
   constexpr bool kTwo = EPI == EPI_SWIGLU;              // two weight sets
@@ -238,13 +243,13 @@ __global__ __launch_bounds__(kThreads, (Cfg<WN, BM>::kBlocks)) void gemm_f32_ker
     for (int m = 0; m < kMG; ++m) acc[f][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const int mg = (t.rows + 15) / 16;
   if (mg == 1)
-    k_loop<WN, BM, 1>(a_src, b_src, n_st, lds, acc);
+    k_loop<WN, BM, NT, 1>(a_src, b_src, n_st, lds, acc);
   else if (BM == 32 || mg == 2)
-    k_loop<WN, BM, 2>(a_src, b_src, n_st, lds, acc);
+    k_loop<WN, BM, NT, 2>(a_src, b_src, n_st, lds, acc);
   else if (mg == 3)
-    k_loop<WN, BM, BM == 32 ? 2 : 3>(a_src, b_src, n_st, lds, acc);
+    k_loop<WN, BM, NT, BM == 32 ? 2 : 3>(a_src, b_src, n_st, lds, acc);
   else
-    k_loop<WN, BM, BM == 32 ? 2 : 4>(a_src, b_src, n_st, lds, acc);
+    k_loop<WN, BM, NT, BM == 32 ? 2 : 4>(a_src, b_src, n_st, lds, acc);
 
   const int wn = wave % WN, wk = wave / WN;
   if (C::kWK > 1) {
@@ -334,19 +339,30 @@ int pick_wn(const GroupedGemmArgs& g, int bm) {
   return g.K % 64 == 0 ? 1 : 2;
 }
 
-template <int WN, int BM, int EPI>
-hipError_t launch_tile(const GroupedGemmArgs& g, hipStream_t s) {
+template <int WN, int BM, int EPI, bool NT>
+hipError_t launch_policy(const GroupedGemmArgs& g, hipStream_t s) {
   using C = Cfg<WN, BM>;
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_f32_kernel<WN, BM, EPI>),
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_f32_kernel<WN, BM, EPI, NT>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, C::kLds);
   (void)attr;
   const int n_col = col_tiles(g, WN);
   const int64_t rows = g.offsets ? max_row_tiles(g.n_assign, g.n_expert, BM) : (g.n_assign + BM - 1) / BM;
   const int64_t blocks = (rows * n_col + 7) / 8 * 8;  // whole rounds of the 8 XCDs
-  hipLaunchKernelGGL((gemm_f32_kernel<WN, BM, EPI>),
+  hipLaunchKernelGGL((gemm_f32_kernel<WN, BM, EPI, NT>),
                      dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(g.ksplit)), dim3(kThreads), C::kLds, s,
                      g, n_col);
   return hipGetLastError();
+}
+
+// The weights go non-temporally up to 64 rows per expert on average, where an
+// expert is mostly one row tile; beyond, its row tiles share them in L2.
+// Measured (DeepSeek-V2-Lite in fp32, whole block, default -> non-temporal):
+// 6 rows 422 -> 378 us, 19 rows 451 -> 408, 47 rows 616 -> 608, 94 rows 1165 ->
+// 1185, 188 rows 1916 -> 1997.
+template <int WN, int BM, int EPI>
+hipError_t launch_tile(const GroupedGemmArgs& g, hipStream_t s) {
+  if (g.n_assign <= 64ll * g.n_expert) return launch_policy<WN, BM, EPI, true>(g, s);
+  return launch_policy<WN, BM, EPI, false>(g, s);
 }
 
 template <int EPI>

@@ -605,7 +605,6 @@ void gemm_stream_kernel(GroupedGemmArgs g, int col_tiles) {
 // Cache policy of the weight loads: non-temporal (each weight byte is read
 // once per launch), as gemm_stream_kernel's, so the weights do not push the
 // token rows and the next kernel's data out of the caches.
-constexpr int kNonTemporal = 2;
 // The Q/K/V kernel's block has two more waves: they compute the RoPE
 // (cos, sin) of each (row, pair) of the block's 16 columns into LDS while
 // the four streaming waves wait on their loads, so the epilogue only

@@ -1215,9 +1215,8 @@ int fmoe_mul_mat_id(const void* packed_w, const float* w_scales, int w_dtype, co
   void* x = at<char>(workspace, L.x);
   void* y = at<char>(workspace, L.y);
   // input [n_in, k*T] -> x [k*T, n_in]: row f = s*T + t (mul_mat_id.mlir:63-90)
-  if (n_in > 0) FMOE_HIP(launch_transpose(input, x, n_in, n, act_dtype, s));
-  FMOE_HIP(launch_permute(ids, static_cast<int>(n), static_cast<int>(n_expert), order, offsets, err,
-                          at<int>(workspace, L.perm.scratch), s));
+  FMOE_HIP(launch_mmid_prepare(input, x, n_in, act_dtype, ids, static_cast<int>(n), static_cast<int>(n_expert), order,
+                               offsets, err, at<int>(workspace, L.perm.scratch), s));
   GroupedGemmArgs g;
   g.a = x;
   g.lda = n_in;
@@ -1242,10 +1241,8 @@ int fmoe_mul_mat_id(const void* packed_w, const float* w_scales, int w_dtype, co
     ScopedTimer t(FMOE_TIMER_MUL_MAT_ID, s);
     FMOE_TRY(run_grouped_gemm(g, s));
   }
-  FMOE_HIP(launch_zero_invalid_rows(ids, static_cast<int>(n), static_cast<int>(n_expert), y,
-                                    act_dtype, n_out, s));
   // y [k*T, n_out] -> out [n_out, k*T] (mul_mat_id.mlir:96-117)
-  FMOE_HIP(launch_transpose(y, out, n, n_out, act_dtype, s));
+  FMOE_HIP(launch_transpose(y, out, n, n_out, act_dtype, ids, static_cast<int>(n_expert), s));
   return ok();
 }
 

@@ -357,36 +357,32 @@ __global__ __launch_bounds__(kThreads) void rms_norm_kernel(const T* x,
   }
 }
 
+// out[c, r] = in[r, c] for an in[rows, cols] matrix.  With ids (mul_mat_id's
+// result) row r is read as zeros where ids[r] is outside [0, n_expert).
 template <typename T>
-__global__ __launch_bounds__(kThreads) void transpose_kernel(const T* __restrict__ in,
-                                                             T* __restrict__ out, int64_t rows,
-                                                             int64_t cols) {
+__global__ __launch_bounds__(kThreads) void transpose_kernel(const T* __restrict__ in, T* __restrict__ out,
+                                                             int64_t rows, int64_t cols, const int* __restrict__ ids,
+                                                             int n_expert) {
   __shared__ T tile[32][33];
   const int64_t c0 = static_cast<int64_t>(blockIdx.x) * 32;
   const int64_t r0 = static_cast<int64_t>(blockIdx.y) * 32;
   const int tx = threadIdx.x & 31;
   const int ty = threadIdx.x >> 5;  // 0..7
+#pragma unroll
   for (int j = ty; j < 32; j += 8) {
     const int64_t r = r0 + j, c = c0 + tx;
-    if (r < rows && c < cols) tile[j][tx] = in[r * cols + c];
+    if (r < rows && c < cols) {
+      const T v = in[r * cols + c];
+      const int e = ids ? ids[r] : 0;
+      tile[j][tx] = e >= 0 && e < n_expert ? v : T(0);
+    }
   }
   __syncthreads();
+#pragma unroll
   for (int j = ty; j < 32; j += 8) {
     const int64_t c = c0 + j, r = r0 + tx;
     if (r < rows && c < cols) out[c * rows + r] = tile[tx][j];
   }
-}
-
-template <typename T>
-__global__ __launch_bounds__(kThreads) void zero_invalid_rows_kernel(const int* __restrict__ ids,
-                                                                     int n_assign, int n_expert,
-                                                                     T* __restrict__ y,
-                                                                     int64_t width) {
-  const int f = blockIdx.x;
-  if (f >= n_assign) return;
-  const int e = ids[f];
-  if (e >= 0 && e < n_expert) return;
-  for (int64_t c = threadIdx.x; c < width; c += kThreads) y[f * width + c] = T(0);
 }
 
 __global__ __launch_bounds__(kThreads) void fill_zero_kernel(uint32_t* __restrict__ p, size_t n) {
@@ -500,29 +496,18 @@ hipError_t launch_rms_norm(const void* x, const void* weight, float eps, void* o
   return hipGetLastError();
 }
 
-hipError_t launch_transpose(const void* in, void* out, int64_t rows, int64_t cols, int dtype,
-                            hipStream_t stream) {
+hipError_t launch_transpose(const void* in, void* out, int64_t rows, int64_t cols, int dtype, const int* ids,
+                            int n_expert, hipStream_t stream) {
   if (rows == 0 || cols == 0) return hipSuccess;
   const dim3 grid(static_cast<unsigned>((cols + 31) / 32), static_cast<unsigned>((rows + 31) / 32));
   if (grid.y > 65535) return hipErrorInvalidValue;
+  if (!ids) n_expert = 1;
   if (dtype == DT_F32)
-    hipLaunchKernelGGL(transpose_kernel<float>, grid, dim3(kThreads), 0, stream,
-                       static_cast<const float*>(in), static_cast<float*>(out), rows, cols);
+    hipLaunchKernelGGL(transpose_kernel<float>, grid, dim3(kThreads), 0, stream, static_cast<const float*>(in),
+                       static_cast<float*>(out), rows, cols, ids, n_expert);
   else
-    hipLaunchKernelGGL(transpose_kernel<bf16_t>, grid, dim3(kThreads), 0, stream,
-                       static_cast<const bf16_t*>(in), static_cast<bf16_t*>(out), rows, cols);
-  return hipGetLastError();
-}
-
-hipError_t launch_zero_invalid_rows(const int* ids, int n_assign, int n_expert, void* y, int dtype,
-                                    int64_t width, hipStream_t stream) {
-  if (n_assign == 0 || width == 0) return hipSuccess;
-  if (dtype == DT_F32)
-    hipLaunchKernelGGL(zero_invalid_rows_kernel<float>, dim3(n_assign), dim3(kThreads), 0, stream,
-                       ids, n_assign, n_expert, static_cast<float*>(y), width);
-  else
-    hipLaunchKernelGGL(zero_invalid_rows_kernel<bf16_t>, dim3(n_assign), dim3(kThreads), 0, stream,
-                       ids, n_assign, n_expert, static_cast<bf16_t*>(y), width);
+    hipLaunchKernelGGL(transpose_kernel<bf16_t>, grid, dim3(kThreads), 0, stream, static_cast<const bf16_t*>(in),
+                       static_cast<bf16_t*>(out), rows, cols, ids, n_expert);
   return hipGetLastError();
 }
 

@@ -801,39 +801,46 @@ __device__ __forceinline__ WaveCtx tile_ctx(const GroupedGemmArgs& g, const Tile
 // rows it has, then the 16 weight blocks) in an 8-deep ring with 6 stages
 // in flight, against 2-3 of the 32 KiB stages in the main loop.  Waves 0-3
 // load token group `wave` and every wave its two weight blocks; one barrier
-// per stage (a buffer is refilled two stages after its last read).  The
-// weights are loaded non-temporally: a thin tile is mostly its expert's only
-// tile, or the last of a few.  Measured (whole block, default -> non-temporal):
-// Mixtral 200 tokens 544 -> 511 us, DeepSeek-V2-Lite 300 tokens 235 -> 221 us,
-// Qwen3 500 and 2043 tokens 212 -> 208 and 336 -> 331 us, Mixtral 4096 level.
-// Not for the main loop's stages: the row tiles of an expert share them in L2
-// (Mixtral 4096 tokens 2345 -> 2618 us).
+// per stage (a buffer is refilled two stages after its last read).  An
+// expert's only row tile loads its weights non-temporally; a thin last tile
+// behind full ones shares them in L2.  Measured (whole block, default ->
+// non-temporal): Mixtral 200 tokens 544 -> 511 us, DeepSeek-V2-Lite 300 tokens
+// 235 -> 221 us, Qwen3 500 and 2043 tokens 212 -> 208 and 336 -> 331 us; on thin
+// last tiles too, the gate projection at Mixtral's 250 rows per expert went
+// 418 -> 456 us, and the main loop's stages lose far more (Mixtral 4096 tokens
+// 2345 -> 2618 us).
 constexpr int kThinRows = 64;
 constexpr int kThinStage = 20 * 1024;
 constexpr int kThinRing = kLds / kThinStage;  // 8
 constexpr int kThinAhead = kThinRing - 2;     // stages in flight
 
+template <bool NT>
 __device__ __forceinline__ void thin_issue(const WaveCtx& c, uint32_t a_off_thin, int kt, int buf) {
   unsigned char* st = c.lds + buf * kThinStage;
   if (c.wave < 4)
     __builtin_amdgcn_global_load_lds(c.a_base + (a_off_thin + static_cast<uint32_t>(kt) * c.a_kstride),
                                      st + c.wave * 1024, 16, 0, 0);
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
-    __builtin_amdgcn_global_load_lds(c.b_base[j] + (static_cast<uint32_t>(kt) * 1024 + c.b_lane),
-                                     st + 4096 + (c.wave * 2 + j) * 1024, 16, 0, kNonTemporal);
+  for (int j = 0; j < 2; ++j) {
+    const unsigned char* src = c.b_base[j] + (static_cast<uint32_t>(kt) * 1024 + c.b_lane);
+    unsigned char* dst = st + 4096 + (c.wave * 2 + j) * 1024;
+    if (NT)
+      __builtin_amdgcn_global_load_lds(src, dst, 16, 0, kNonTemporal);
+    else
+      __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
+  }
 }
 
-template <int NSETS>
+template <int NSETS, bool NT>
 __device__ __forceinline__ void thin_k_loop(const WaveCtx& c, uint32_t a_off_thin, int rows, f32x4_t (&acc)[8][4]) {
   const int KT = c.KT;
   const bool active = c.wm * 16 < rows;  // this wave pair's row group holds rows
-  for (int kt = 0; kt < kThinAhead && kt < KT; ++kt) thin_issue(c, a_off_thin, kt, kt);
+  for (int kt = 0; kt < kThinAhead && kt < KT; ++kt) thin_issue<NT>(c, a_off_thin, kt, kt);
   for (int kt = 0; kt < KT; ++kt) {
     // Refill the buffer read two stages ago, then wait for stage kt (loads
     // per stage: 3 for waves 0-3, 2 for the others).
     if (kt + kThinAhead < KT) {
-      thin_issue(c, a_off_thin, kt + kThinAhead, (kt + kThinAhead) % kThinRing);
+      thin_issue<NT>(c, a_off_thin, kt + kThinAhead, (kt + kThinAhead) % kThinRing);
       if (c.wave < 4)
         __builtin_amdgcn_s_waitcnt(wait_vm(3 * kThinAhead, false));
       else
@@ -966,7 +973,11 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled256_kernel(GroupedGemmA
   } else {
     if (!A8 && kThin && ti.rows <= kThinRows) {
       const int64_t kb_first = split_boundary(static_cast<int>(g.K / 32), g.ksplit, split, g.ksplit_first64);
-      thin_k_loop<NSETS>(c, a_group_offset(g, ti, wave & 3, lane, kb_first), ti.rows, acc);
+      const uint32_t a_off_thin = a_group_offset(g, ti, wave & 3, lane, kb_first);
+      if (g.offsets[ti.expert + 1] - g.offsets[ti.expert] == ti.rows)  // the expert's only row tile
+        thin_k_loop<NSETS, true>(c, a_off_thin, ti.rows, acc);
+      else
+        thin_k_loop<NSETS, false>(c, a_off_thin, ti.rows, acc);
     } else {
       k_issue_range<NSETS>(c, 0, 4);
       run_k_body<NSETS, A8>(c, acc, ti.rows);

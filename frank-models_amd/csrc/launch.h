@@ -307,13 +307,16 @@ hipError_t launch_combine(const void* y, int y_dtype, const void* residual, void
 // out[r, :] = (x[r, :] / sqrt(mean(x[r, :]^2) + eps)) * weight, fp32 arithmetic.
 hipError_t launch_rms_norm(const void* x, const void* weight, float eps, void* out, int64_t n_rows,
                            int n_embd, int dtype, hipStream_t stream);
-// out[c, r] = in[r, c] for an in[rows, cols] matrix (same dtype).
-hipError_t launch_transpose(const void* in, void* out, int64_t rows, int64_t cols,
-                            int dtype, hipStream_t stream);
-// Zero rows f of y[n_assign, width] whose id is outside [0, n_expert).
-hipError_t launch_zero_invalid_rows(const int* ids, int n_assign, int n_expert,
-                                    void* y, int dtype, int64_t width,
-                                    hipStream_t stream);
+// out[c, r] = in[r, c] for an in[rows, cols] matrix (same dtype); with ids
+// (may be null), rows r whose ids[r] is outside [0, n_expert) read as zeros.
+hipError_t launch_transpose(const void* in, void* out, int64_t rows, int64_t cols, int dtype, const int* ids,
+                            int n_expert, hipStream_t stream);
+// mul_mat_id's operands: x [n, n_in] = input [n_in, n] transposed (same
+// dtype), and the permutation of its n ids (as launch_permute), in one launch
+// up to kPermuteChunk ids.
+hipError_t launch_mmid_prepare(const void* input, void* x, int64_t n_in, int dtype, const int* ids, int n,
+                               int n_expert, int* order, int* offsets, int* err_count, int* scratch,
+                               hipStream_t stream);
 hipError_t launch_fill_zero(void* p, size_t bytes, hipStream_t stream);
 // Rows of src [*, n_cols] bf16 (row p = src row order[p] % n_tokens, or row p
 // when order is null), quantised to e4m3 with one scale per row: scale[p] =

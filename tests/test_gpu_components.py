@@ -406,3 +406,28 @@ def test_row_quantizer_codes_match_the_oracle(fm, two_terms):
         np.testing.assert_array_equal(_unblock_e4m3(lo.cpu().numpy(), n_rows, n_cols), rl)
     else:
         assert not lo.any()
+
+
+@pytest.mark.parametrize("T", [8, 700])
+def test_mul_mat_id_device_ids_checked_apart(fm, T):
+    """Weights large enough that the ids are checked on a launch and a stream of
+    their own: out-of-range device ids still raise at the call, on the default
+    and on another stream, and the calls around it are unaffected.  T = 700
+    with 4 slots: above the one-block permutation's 2048 ids."""
+    n, E, k = 2048, 32, 4  # 256 MB of bf16 weights, every expert routed to
+    g = torch.Generator(device="cuda").manual_seed(3)
+    w = fm.pack_expert_weights(torch.randn((n, n, E), device="cuda", generator=g).bfloat16())
+    x = torch.randn((n, k, T), device="cuda", generator=g).bfloat16()
+    ids = torch.rand((T, E), device="cuda", generator=g).topk(k, dim=1).indices.T.to(torch.int32).contiguous()
+    good = fm.mul_mat_id(w, x, ids)
+    for stream in (torch.cuda.current_stream(), torch.cuda.Stream()):
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            for bad in (E, -1):
+                wrong = ids.clone()
+                wrong[k - 1, T - 1] = bad
+                with pytest.raises(IndexError, match="1 expert id"):
+                    fm.mul_mat_id(w, x, wrong)
+            again = fm.mul_mat_id(w, x, ids)
+        torch.cuda.synchronize()
+        assert torch.equal(good, again)

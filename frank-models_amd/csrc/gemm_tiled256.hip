@@ -18,8 +18,8 @@
 // from global memory (global_load_lds_dwordx4, no staging registers).  The
 // two waves of each SIMD take turns: one multiplies two stages while the
 // other reads its next fragments and issues the loads of a stage two to
-// three stages ahead (k_body).  Tiles of at most 64 rows take a loop of
-// their own (thin_k_loop); fp8 weights take k_loop_f8.
+// three stages ahead (k_body).  Tiles of at most 128 rows (fp8 weights: 64)
+// take a loop of their own (narrow_k_loop); fp8 weights take k_loop_f8.
 //
 // Tile order: each XCD works through a contiguous range of the tiles
 // (sched_tile), or, for GEMMs of 16 or more column tiles, through a list
@@ -50,10 +50,7 @@ constexpr int kLds = kRing * kStage;         // 160 KiB
 // fp8 weights: 64-input stages (A as two 32-input halves in the bf16 layout,
 // then 16 fp8 weight blocks of 16 rows x 64 inputs), 3-deep ring.
 constexpr int kStagesF8 = 3;
-constexpr int kStageF8 = 2 * kAStage + kBStage;  // 48 KiB
-constexpr int kLdsF8 = kStagesF8 * kStageF8;     // 144 KiB
 constexpr int kGroupN = 4;                   // column tiles swept together
-constexpr bool kThin = true;                 // tiles of <= 64 rows take the thin loop (bf16)
 
 __device__ __forceinline__ f32x4_t mfma16(const u32x4_t a, const u32x4_t b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
@@ -565,18 +562,31 @@ __device__ __forceinline__ void k_body(const WaveCtx& c, f32x4_t (&acc)[8][4]) {
 // row set d & 1; d = 4, 5: weight blocks).
 // With two-term e4m3 activations (X2) the A halves are the stage's 64-input
 // piece of the hi codes (h = 0) and of the lo codes (h = 1).
-template <bool X2>
+// HALF: tiles of at most 128 rows, whose stages hold 8 row groups (each wave
+// loads one) in a 5-deep ring; c.a_off[0] is then row group `wave`.
+template <bool HALF>
+struct StageF8 {
+  static constexpr int kAHalf = HALF ? kAStage / 2 : kAStage;  // one A half
+  static constexpr int kBytes = 2 * kAHalf + kBStage;
+  static constexpr int kRing = HALF ? 5 : kStagesF8;
+  static constexpr int kLoads = HALF ? 4 : 6;                  // per wave
+};
+
+template <bool X2, bool HALF>
 __device__ __forceinline__ void issue_one_f8(const WaveCtx& c, int kt, int buf, int d) {
-  unsigned char* st = c.lds + buf * kStageF8;
-  if (d < 4) {
-    const int h = d >> 1, j = d & 1;
+  using S = StageF8<HALF>;
+  constexpr int kALoads = S::kLoads - 2;
+  unsigned char* st = c.lds + buf * S::kBytes;
+  if (d < kALoads) {
+    const int h = HALF ? d : d >> 1, j = HALF ? 0 : d & 1;
     const uint32_t src = X2 ? h * c.a_plane + c.a_off[j] + static_cast<uint32_t>(kt) * c.a_kstride
                             : c.a_off[j] + static_cast<uint32_t>(2 * kt + h) * c.a_kstride;
-    __builtin_amdgcn_global_load_lds(c.a_base + src, st + h * kAStage + (c.wave * 2 + j) * 1024, 16, 0, 0);
+    unsigned char* dst = st + h * S::kAHalf + (HALF ? c.wave : c.wave * 2 + j) * 1024;
+    __builtin_amdgcn_global_load_lds(c.a_base + src, dst, 16, 0, 0);
   } else {
-    const int j = d - 4;
-    __builtin_amdgcn_global_load_lds(c.b_base[j] + (static_cast<uint32_t>(kt) * 1024 + c.b_lane),
-                                     st + 2 * kAStage + (c.wave * 2 + j) * 1024, 16, 0, 0);
+    const int j = d - kALoads;
+    unsigned char* dst = st + 2 * S::kAHalf + (c.wave * 2 + j) * 1024;
+    __builtin_amdgcn_global_load_lds(c.b_base[j] + (static_cast<uint32_t>(kt) * 1024 + c.b_lane), dst, 16, 0, 0);
   }
 }
 
@@ -597,24 +607,25 @@ __device__ __forceinline__ u32x4_t convert_frag(const u32x4_t q) {
   return f8x8_to_bf16x8(q[2 * H], q[2 * H + 1]);
 }
 
-// This wave's 6 loads of fp8 stage kt (its share) into buffer buf.
-template <bool X2>
+// This wave's loads of fp8 stage kt (its share) into buffer buf.
+template <bool X2, bool HALF>
 __device__ __forceinline__ void issue_share_f8(const WaveCtx& c, int kt, int buf) {
 #pragma unroll
-  for (int d = 0; d < 6; ++d) issue_one_f8<X2>(c, kt, buf, d);
+  for (int d = 0; d < StageF8<HALF>::kLoads; ++d) issue_one_f8<X2, HALF>(c, kt, buf, d);
 }
 
 // A fragments of both 32-input halves and the 8 raw fp8 weight fragments of
 // the stage in buffer buf.
-template <int NM, int NSETS>
+template <int NM, int NSETS, bool HALF>
 __device__ __forceinline__ void read_stage_f8(const WaveCtx& c, int buf, u32x4_t (&fa)[2][4], u32x4_t (&fq)[8]) {
-  const unsigned char* st = c.lds + buf * kStageF8;
+  using S = StageF8<HALF>;
+  const unsigned char* st = c.lds + buf * S::kBytes;
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int m = 0; m < NM; ++m) fa[h][m] = read_a_frag(c, st + h * kAStage, m);
+    for (int m = 0; m < NM; ++m) fa[h][m] = read_a_frag(c, st + h * S::kAHalf, m);
 #pragma unroll
-  for (int n = 0; n < 8; ++n) fq[n] = read_b_frag<NSETS>(c, st + 2 * kAStage, n);
+  for (int n = 0; n < 8; ++n) fq[n] = read_b_frag<NSETS>(c, st + 2 * S::kAHalf, n);
 }
 
 // The 64 MFMAs of one fp8 stage, half by half; weight fragment n+1's codes
@@ -649,30 +660,32 @@ __device__ __forceinline__ void multiply_f8(f32x4_t (&acc)[8][4], const u32x4_t 
 }
 
 // K loop for fp8 weights: the bf16 loop's ping-pong between wave groups G0
-// (waves 0-3) and G1 (waves 4-7), one 64-input stage per slot, a 3-deep ring
-// (R = kStagesF8), and each wave loading its own share (6 loads) of a stage.
+// (waves 0-3) and G1 (waves 4-7), one 64-input stage per slot, a ring of R
+// stages (3; 5 for tiles of at most 128 rows), and each wave loading its own
+// share of a stage.
 //   Slot 2k:   G0 multiplies stage k; G1 reads stage k and loads stage k+2.
 //   Slot 2k+1: G1 multiplies stage k; G0 reads stage k+1 and loads stage k+3.
-// Every memory slot ends with lgkmcnt(0) and vmcnt(6): only the share just
-// issued may be in flight, so G1 has stage k+1 and G0 stage k+2 complete,
+// (with R = 3; R - 1 and R stages on in general).
+// Every memory slot ends with lgkmcnt(0) and a wait that leaves the R - 2
+// youngest shares in flight, so G1 has stage k+1 and G0 stage k+2 complete,
 // each ahead of the barrier before its first reader.  The buffer a load
 // refills held stage k-1 (G1, last read in slot 2k-2) or stage k (G0, last
 // read in slot 2k); the other buffers hold stages being read or still
 // landing.  Loads past the last stage are not issued (those slots wait for
 // everything instead); the prologue re-reads the last stage into buffers
 // that are never read when K has fewer stages than the ring.
-template <int NM, int NSETS, int G, bool X2>
+template <int NM, int NSETS, int G, bool X2, bool HALF>
 __device__ __forceinline__ void k_loop_f8(const WaveCtx& c, f32x4_t (&acc)[8][4]) {
-  constexpr int R = kStagesF8;
+  constexpr int R = StageF8<HALF>::kRing, kLoads = StageF8<HALF>::kLoads;
   const int KT = c.KT;
   u32x4_t fa[2][4], fq[8];
 #pragma unroll
-  for (int s = 0; s < (G == 0 ? R : R - 1); ++s) issue_share_f8<X2>(c, s < KT ? s : KT - 1, s);
-  __builtin_amdgcn_s_waitcnt(wait_vm(6 * (G == 0 ? R - 1 : R - 2), false));
+  for (int s = 0; s < (G == 0 ? R : R - 1); ++s) issue_share_f8<X2, HALF>(c, s < KT ? s : KT - 1, s);
+  __builtin_amdgcn_s_waitcnt(wait_vm(kLoads * (G == 0 ? R - 1 : R - 2), false));
   asm volatile("s_barrier" ::: "memory");
   if constexpr (G == 0) {
-    if constexpr (NM > 0) read_stage_f8<NM, NSETS>(c, 0, fa, fq);
-    __builtin_amdgcn_s_waitcnt(wait_vm(6 * (R - 2), true));
+    if constexpr (NM > 0) read_stage_f8<NM, NSETS, HALF>(c, 0, fa, fq);
+    __builtin_amdgcn_s_waitcnt(wait_vm(kLoads * (R - 2), true));
   }
   asm volatile("s_barrier" ::: "memory");
 
@@ -688,11 +701,11 @@ __device__ __forceinline__ void k_loop_f8(const WaveCtx& c, f32x4_t (&acc)[8][4]
       asm volatile("s_barrier" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (NM > 0)
-        if (kt + 1 < KT) read_stage_f8<NM, NSETS>(c, rd, fa, fq);
+        if (kt + 1 < KT) read_stage_f8<NM, NSETS, HALF>(c, rd, fa, fq);
       if (kt + R < KT) {
-        issue_share_f8<X2>(c, kt + R, wr);
+        issue_share_f8<X2, HALF>(c, kt + R, wr);
         __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(wait_vm(6 * (R - 2), true));
+        __builtin_amdgcn_s_waitcnt(wait_vm(kLoads * (R - 2), true));
       } else {
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(wait_vm(0, true));
@@ -700,11 +713,11 @@ __device__ __forceinline__ void k_loop_f8(const WaveCtx& c, f32x4_t (&acc)[8][4]
       asm volatile("s_barrier" ::: "memory");
     } else {
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (NM > 0) read_stage_f8<NM, NSETS>(c, rd, fa, fq);
+      if constexpr (NM > 0) read_stage_f8<NM, NSETS, HALF>(c, rd, fa, fq);
       if (kt + R - 1 < KT) {
-        issue_share_f8<X2>(c, kt + R - 1, wr);
+        issue_share_f8<X2, HALF>(c, kt + R - 1, wr);
         __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(wait_vm(6 * (R - 2), true));
+        __builtin_amdgcn_s_waitcnt(wait_vm(kLoads * (R - 2), true));
       } else {
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(wait_vm(0, true));
@@ -721,6 +734,32 @@ __device__ __forceinline__ void k_loop_f8(const WaveCtx& c, f32x4_t (&acc)[8][4]
     wr = wr + 1 == R ? 0 : wr + 1;
   }
   __builtin_amdgcn_s_waitcnt(kWaitVm0);
+}
+
+// The fp8-weight K loop of a tile with `rows` rows: this wave's active 16-row
+// groups (wm, wm + 4, ... below ceil(rows / 16), at most MAXM) select the
+// specialisation.
+template <int MAXM, int NSETS, bool X2, bool HALF>
+__device__ __forceinline__ void run_k_f8(const WaveCtx& c, f32x4_t (&acc)[8][4], int rows) {
+  const int groups = (rows + 15) >> 4;
+  const int nm = groups > c.wm ? min(MAXM, (groups - c.wm + 3) >> 2) : 0;
+  if (c.wave < 4) {
+    switch (nm) {
+      case 4: if constexpr (MAXM == 4) k_loop_f8<4, NSETS, 0, X2, HALF>(c, acc); break;
+      case 3: if constexpr (MAXM == 4) k_loop_f8<3, NSETS, 0, X2, HALF>(c, acc); break;
+      case 2: k_loop_f8<2, NSETS, 0, X2, HALF>(c, acc); break;
+      case 1: k_loop_f8<1, NSETS, 0, X2, HALF>(c, acc); break;
+      default: k_loop_f8<0, NSETS, 0, X2, HALF>(c, acc); break;
+    }
+  } else {
+    switch (nm) {
+      case 4: if constexpr (MAXM == 4) k_loop_f8<4, NSETS, 1, X2, HALF>(c, acc); break;
+      case 3: if constexpr (MAXM == 4) k_loop_f8<3, NSETS, 1, X2, HALF>(c, acc); break;
+      case 2: k_loop_f8<2, NSETS, 1, X2, HALF>(c, acc); break;
+      case 1: k_loop_f8<1, NSETS, 1, X2, HALF>(c, acc); break;
+      default: k_loop_f8<0, NSETS, 1, X2, HALF>(c, acc); break;
+    }
+  }
 }
 
 // Byte offset (from the A base) of this lane's 16-byte piece of 16-row
@@ -795,35 +834,61 @@ __device__ __forceinline__ WaveCtx tile_ctx(const GroupedGemmArgs& g, const Tile
   return c;
 }
 
-// ---- Thin tiles (bf16, at most 64 rows: one 16-row group per wave pair).
+// ---- Narrow tiles (bf16 activations; at most 128 rows, with fp8 weights 64).
 // Such a tile is bound by how many weight bytes are in flight, not by its
-// few MFMAs, so it runs its own loop: 20 KiB stages (the 4 KiB of token
-// rows it has, then the 16 weight blocks) in an 8-deep ring with 6 stages
-// in flight, against 2-3 of the 32 KiB stages in the main loop.  Waves 0-3
-// load token group `wave` and every wave its two weight blocks; one barrier
-// per stage (a buffer is refilled two stages after its last read).  An
-// expert's only row tile loads its weights non-temporally; a thin last tile
-// behind full ones shares them in L2.  Measured (whole block, default ->
+// MFMAs, so it runs its own loop: stages that hold only the token rows it has
+// (MG = 1: 64, MG = 2: 128) beside the 16 weight blocks, in as deep a ring as
+// the LDS holds (bf16 8 or 6 stages of 20 or 24 KiB; fp8 weights, 64 inputs a
+// stage, 6 of 24 KiB) with all but two of them in flight, against 2-3 stages
+// of the main loops.  A wave loads its share of the token groups and two
+// weight blocks; one barrier per stage (a buffer is refilled two stages after
+// its last read).  Measured (whole block, before -> with this loop and the
+// loads below): bf16 Mixtral 64 / 160 / 333 / 480 tokens 531 -> 478, 544 -> 505,
+// 571 -> 538, 594 -> 580 us; Qwen3 500 / 2043 tokens 219 -> 204, 350 -> 335 us;
+// DeepSeek-V2-Lite 300 / 1100 tokens 234 -> 220, 269 -> 258 us; fp8 Mixtral 40 /
+// 120 / 200 tokens 293 -> 263, 308 -> 279, 341 -> 307 us.  fp8 weights with 65-128
+// rows are no gain here (Mixtral 333 tokens 356 -> 407 us: every wave converts
+// the same 8 fragments in step and nothing multiplies meanwhile); they keep
+// the ping-pong of k_loop_f8 with a 5-deep ring of smaller stages (two 8 KiB
+// halves of token rows instead of 16 KiB), 369 -> 366 us there, and Mixtral x2
+// 300 tokens 391 -> 383 us.
+// An expert's only row tile loads its weights non-temporally; a narrow last
+// tile behind full ones shares them in L2.  Measured (whole block, default ->
 // non-temporal): Mixtral 200 tokens 544 -> 511 us, DeepSeek-V2-Lite 300 tokens
 // 235 -> 221 us, Qwen3 500 and 2043 tokens 212 -> 208 and 336 -> 331 us; on thin
 // last tiles too, the gate projection at Mixtral's 250 rows per expert went
 // 418 -> 456 us, and the main loop's stages lose far more (Mixtral 4096 tokens
 // 2345 -> 2618 us).
-constexpr int kThinRows = 64;
-constexpr int kThinStage = 20 * 1024;
-constexpr int kThinRing = kLds / kThinStage;  // 8
-constexpr int kThinAhead = kThinRing - 2;     // stages in flight
+constexpr int kNarrowRows = 128;
+constexpr int kNarrowRowsF8 = 64;
 
-template <bool NT>
-__device__ __forceinline__ void thin_issue(const WaveCtx& c, uint32_t a_off_thin, int kt, int buf) {
-  unsigned char* st = c.lds + buf * kThinStage;
-  if (c.wave < 4)
-    __builtin_amdgcn_global_load_lds(c.a_base + (a_off_thin + static_cast<uint32_t>(kt) * c.a_kstride),
-                                     st + c.wave * 1024, 16, 0, 0);
+template <int MG, bool F8>
+struct Narrow {
+  static constexpr int kHalves = F8 ? 2 : 1;               // 32-input halves of a stage
+  static constexpr int kHalfB = MG * 4 * 1024;
+  static constexpr int kABytes = kHalves * kHalfB;
+  static constexpr int kStageB = kABytes + kBStage;
+  static constexpr int kRingN = kLds / kStageB;
+  static constexpr int kAhead = kRingN - 2;                // stages in flight
+  static constexpr int kLoads = 3;                         // per wave; 2 of waves 4-7 with 4 token groups
+  static_assert(MG * kHalves <= 2, "one token group per wave");
+};
+
+// a_off: this wave's token group (wave % (4 MG)) in stage 0.
+template <int MG, bool F8, bool NT>
+__device__ __forceinline__ void narrow_issue(const WaveCtx& c, uint32_t a_off, int kt, int buf) {
+  using W = Narrow<MG, F8>;
+  unsigned char* st = c.lds + buf * W::kStageB;
+  // fp8 with 4 groups: waves 0-3 load half 0, waves 4-7 half 1
+  const int half = F8 ? c.wave >> 2 : 0;
+  const uint32_t piece = static_cast<uint32_t>(F8 ? 2 * kt + half : kt);
+  unsigned char* a_dst = st + half * W::kHalfB + (MG == 1 ? c.wave & 3 : c.wave) * 1024;
+  const unsigned char* a_src = c.a_base + (a_off + piece * c.a_kstride);
+  if (F8 || MG == 2 || c.wave < 4) __builtin_amdgcn_global_load_lds(a_src, a_dst, 16, 0, 0);
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const unsigned char* src = c.b_base[j] + (static_cast<uint32_t>(kt) * 1024 + c.b_lane);
-    unsigned char* dst = st + 4096 + (c.wave * 2 + j) * 1024;
+    unsigned char* dst = st + W::kABytes + (c.wave * 2 + j) * 1024;
     if (NT)
       __builtin_amdgcn_global_load_lds(src, dst, 16, 0, kNonTemporal);
     else
@@ -831,38 +896,73 @@ __device__ __forceinline__ void thin_issue(const WaveCtx& c, uint32_t a_off_thin
   }
 }
 
-template <int NSETS, bool NT>
-__device__ __forceinline__ void thin_k_loop(const WaveCtx& c, uint32_t a_off_thin, int rows, f32x4_t (&acc)[8][4]) {
+template <int NSETS, int MG, bool F8, bool NT>
+__device__ __forceinline__ void narrow_k_loop(const WaveCtx& c, uint32_t a_off, int rows, f32x4_t (&acc)[8][4]) {
+  using W = Narrow<MG, F8>;
   const int KT = c.KT;
-  const bool active = c.wm * 16 < rows;  // this wave pair's row group holds rows
-  for (int kt = 0; kt < kThinAhead && kt < KT; ++kt) thin_issue<NT>(c, a_off_thin, kt, kt);
+  // this wave pair's row groups wm (and wm + 4) that hold rows
+  const bool active0 = c.wm * 16 < rows, active1 = MG == 2 && (c.wm + 4) * 16 < rows;
+  for (int kt = 0; kt < W::kAhead && kt < KT; ++kt) narrow_issue<MG, F8, NT>(c, a_off, kt, kt);
   for (int kt = 0; kt < KT; ++kt) {
-    // Refill the buffer read two stages ago, then wait for stage kt (loads
-    // per stage: 3 for waves 0-3, 2 for the others).
-    if (kt + kThinAhead < KT) {
-      thin_issue<NT>(c, a_off_thin, kt + kThinAhead, (kt + kThinAhead) % kThinRing);
-      if (c.wave < 4)
-        __builtin_amdgcn_s_waitcnt(wait_vm(3 * kThinAhead, false));
+    // Refill the buffer read two stages ago, then wait for stage kt (and for
+    // this wave's reads of stage kt - 1, whose buffer the next trip refills).
+    if (kt + W::kAhead < KT) {
+      narrow_issue<MG, F8, NT>(c, a_off, kt + W::kAhead, (kt + W::kAhead) % W::kRingN);
+      if (F8 || MG == 2 || c.wave < 4)
+        __builtin_amdgcn_s_waitcnt(wait_vm(W::kLoads * W::kAhead, true));
       else
-        __builtin_amdgcn_s_waitcnt(wait_vm(2 * kThinAhead, false));
+        __builtin_amdgcn_s_waitcnt(wait_vm(2 * W::kAhead, true));
     } else {
-      __builtin_amdgcn_s_waitcnt(kWaitVm0);
+      __builtin_amdgcn_s_waitcnt(wait_vm(0, true));
     }
     asm volatile("s_barrier" ::: "memory");
-    if (active) {
-      const unsigned char* st = c.lds + (kt % kThinRing) * kThinStage;
-      const u32x4_t fa = *reinterpret_cast<const u32x4_t*>(st + c.wm * 1024 + c.a_lane);
-      u32x4_t fb[8];
+    if (active0) {
+      const unsigned char* st = c.lds + (kt % W::kRingN) * W::kStageB;
+      u32x4_t fa[2][2], fb[8];
+#pragma unroll
+      for (int h = 0; h < W::kHalves; ++h)
+#pragma unroll
+        for (int m = 0; m < MG; ++m)
+          fa[h][m] = *reinterpret_cast<const u32x4_t*>(st + h * W::kHalfB + (c.wm + 4 * m) * 1024 + c.a_lane);
 #pragma unroll
       for (int n = 0; n < 8; ++n) {
         const int rb = NSETS == 2 ? ((n >> 2) * 8 + c.wn * 4 + (n & 3)) : (c.wn * 8 + n);
-        fb[n] = *reinterpret_cast<const u32x4_t*>(st + 4096 + rb * 1024 + c.b_lane);
+        fb[n] = *reinterpret_cast<const u32x4_t*>(st + W::kABytes + rb * 1024 + c.b_lane);
       }
 #pragma unroll
-      for (int n = 0; n < 8; ++n) acc[n][0] = mfma16(fb[n], fa, acc[n][0]);
+      for (int n = 0; n < 8; ++n) {
+        const u32x4_t w0 = F8 ? convert_frag<0>(fb[n]) : fb[n];
+        const u32x4_t w1 = F8 ? convert_frag<1>(fb[n]) : fb[n];
+        acc[n][0] = mfma16(w0, fa[0][0], acc[n][0]);
+        if (F8) acc[n][0] = mfma16(w1, fa[1][0], acc[n][0]);
+        if (MG == 2 && active1) {
+          acc[n][1] = mfma16(w0, fa[0][MG - 1], acc[n][1]);
+          if (F8) acc[n][1] = mfma16(w1, fa[1][MG - 1], acc[n][1]);
+        }
+      }
     }
   }
   __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
+}
+
+// The narrow loop of tile ti whose A piece 0 is kb_first.
+template <int NSETS, bool F8>
+__device__ __forceinline__ void run_narrow(const GroupedGemmArgs& g, const TileInfo& ti, const WaveCtx& c, int lane,
+                                           int64_t kb_first, f32x4_t (&acc)[8][4]) {
+  const bool only = g.offsets[ti.expert + 1] - g.offsets[ti.expert] == ti.rows;  // the expert's only row tile
+  if (ti.rows <= 64) {
+    const uint32_t a_off = a_group_offset(g, ti, c.wave & 3, lane, kb_first);
+    if (only)
+      narrow_k_loop<NSETS, 1, F8, true>(c, a_off, ti.rows, acc);
+    else
+      narrow_k_loop<NSETS, 1, F8, false>(c, a_off, ti.rows, acc);
+  } else if constexpr (!F8) {
+    const uint32_t a_off = a_group_offset(g, ti, c.wave, lane, kb_first);
+    if (only)
+      narrow_k_loop<NSETS, 2, F8, true>(c, a_off, ti.rows, acc);
+    else
+      narrow_k_loop<NSETS, 2, F8, false>(c, a_off, ti.rows, acc);
+  }
 }
 
 // The bf16 / fp8-activation K loop of a tile with `rows` rows, after its
@@ -950,38 +1050,25 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled256_kernel(GroupedGemmA
 
   EpiRows er;
   epi_rows_first<EPI>(g, ti, er);
-  if constexpr (F8 && (!A8 || X2)) {
-    const int groups = (ti.rows + 15) >> 4;
-    const int nm = groups > c.wm ? min(4, (groups - c.wm + 3) >> 2) : 0;
-    if (wave < 4) {
-      switch (nm) {
-        case 4: k_loop_f8<4, NSETS, 0, X2>(c, acc); break;
-        case 3: k_loop_f8<3, NSETS, 0, X2>(c, acc); break;
-        case 2: k_loop_f8<2, NSETS, 0, X2>(c, acc); break;
-        case 1: k_loop_f8<1, NSETS, 0, X2>(c, acc); break;
-        default: k_loop_f8<0, NSETS, 0, X2>(c, acc); break;
-      }
+  if (!A8 && ti.rows <= (F8 ? kNarrowRowsF8 : kNarrowRows)) {
+    // first 32-input A piece of this block's K range
+    const int kblocks = static_cast<int>(g.K / (F8 ? 64 : 32));
+    const int64_t kb_first = static_cast<int64_t>(split_boundary(kblocks, g.ksplit, split, g.ksplit_first64)) * (F8 ? 2 : 1);
+    run_narrow<NSETS, F8>(g, ti, c, lane, kb_first, acc);
+  } else if constexpr (F8 && (!A8 || X2)) {
+    if (ti.rows <= kNarrowRows) {
+      // A pieces of the K range's first stage: two 32-input bf16 pieces a
+      // stage, or one 64-input piece of each term
+      const int k_first = split_boundary(static_cast<int>(g.K / 64), g.ksplit, split, g.ksplit_first64);
+      WaveCtx h = c;
+      h.a_off[0] = a_group_offset(g, ti, wave, lane, static_cast<int64_t>(k_first) * (X2 ? 1 : 2));
+      run_k_f8<2, NSETS, X2, true>(h, acc, ti.rows);
     } else {
-      switch (nm) {
-        case 4: k_loop_f8<4, NSETS, 1, X2>(c, acc); break;
-        case 3: k_loop_f8<3, NSETS, 1, X2>(c, acc); break;
-        case 2: k_loop_f8<2, NSETS, 1, X2>(c, acc); break;
-        case 1: k_loop_f8<1, NSETS, 1, X2>(c, acc); break;
-        default: k_loop_f8<0, NSETS, 1, X2>(c, acc); break;
-      }
+      run_k_f8<4, NSETS, X2, false>(c, acc, ti.rows);
     }
   } else {
-    if (!A8 && kThin && ti.rows <= kThinRows) {
-      const int64_t kb_first = split_boundary(static_cast<int>(g.K / 32), g.ksplit, split, g.ksplit_first64);
-      const uint32_t a_off_thin = a_group_offset(g, ti, wave & 3, lane, kb_first);
-      if (g.offsets[ti.expert + 1] - g.offsets[ti.expert] == ti.rows)  // the expert's only row tile
-        thin_k_loop<NSETS, true>(c, a_off_thin, ti.rows, acc);
-      else
-        thin_k_loop<NSETS, false>(c, a_off_thin, ti.rows, acc);
-    } else {
-      k_issue_range<NSETS>(c, 0, 4);
-      run_k_body<NSETS, A8>(c, acc, ti.rows);
-    }
+    k_issue_range<NSETS>(c, 0, 4);
+    run_k_body<NSETS, A8>(c, acc, ti.rows);
   }
   epi_rows_second<EPI>(g, ti, er);
 
@@ -1001,7 +1088,7 @@ hipError_t launch_t(const GroupedGemmArgs& g_in, hipStream_t s) {
   GroupedGemmArgs g = g_in;
   g.ksplit_first64 = gemm_tiled256_split_first64(g);
   if (g.tile_table && gemm_tiled256_table_bytes(g) == 0) g.tile_table = nullptr;
-  constexpr int lds_bytes = F8 && (!A8 || X2) ? kLdsF8 : kLds;
+  constexpr int lds_bytes = kLds;
   static const bool configured = [] {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiled256_kernel<EPI, NSETS, F8, A8, X2>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);

@@ -18,8 +18,8 @@
 // from global memory (global_load_lds_dwordx4, no staging registers).  The
 // two waves of each SIMD take turns: one multiplies two stages while the
 // other reads its next fragments and issues the loads of a stage two to
-// three stages ahead (k_body).  Tiles of at most 128 rows (fp8 weights: 64)
-// take a loop of their own (narrow_k_loop); fp8 weights take k_loop_f8.
+// three stages ahead (k_body).  Tiles of at most 128 rows take
+// a loop of their own (narrow_k_loop); fp8 weights take k_loop_f8.
 //
 // Tile order: each XCD works through a contiguous range of the tiles
 // (sched_tile), or, for GEMMs of 16 or more column tiles, through a list
@@ -283,17 +283,20 @@ __device__ __forceinline__ void epi_rows_second(const GroupedGemmArgs& g, const 
   }
 }
 
-template <int EPI, int NSETS, bool F8, bool A8, bool OUT_F32>
+// HALF: a tile of at most 128 rows whose waves are laid 2 x 4 (StageF8).
+template <int EPI, int NSETS, bool F8, bool A8, bool OUT_F32, bool HALF>
 __device__ __forceinline__ void epilogue(const GroupedGemmArgs& g, const TileInfo& ti, int split, int64_t n0,
                                          int wm, int wn, int lane, unsigned char* lds, const f32x4_t (&acc)[8][4],
                                          const EpiRows& er) {
-  constexpr int kFrags = NSETS == 2 ? 4 : 8;       // output fragments per wave
+  constexpr int kFrags = (NSETS == 2 ? 4 : 8) / (HALF ? 2 : 1);  // output fragments per wave
+  constexpr int kGroupStep = HALF ? 2 : 4;         // between a wave's 16-row groups
+  constexpr int kPassGroups = 8 / kGroupStep;      // its groups per pass of 128 rows
   constexpr int kEsz = OUT_F32 ? 4 : 2;
   constexpr int kRowBytes = (NSETS == 2 ? kBN / 2 : kBN) * kEsz;
   constexpr int kPitch = kRowBytes + 16;
   constexpr int kChunks = kRowBytes / 16;          // 16-byte chunks per row
   const int64_t N = g.N;
-  const int colw = (NSETS == 2 ? wn * 64 : wn * 128) + 4 * (lane >> 4);
+  const int colw = wn * kFrags * 16 + 4 * (lane >> 4);
   constexpr bool kScatter = EPI != EPI_SWIGLU;
   constexpr bool kWeighted = EPI == EPI_SCATTER_WEIGHTED;
   int* t_order = reinterpret_cast<int*>(lds + 128 * kPitch);           // [256]
@@ -313,7 +316,7 @@ __device__ __forceinline__ void epilogue(const GroupedGemmArgs& g, const TileInf
   if constexpr (A8) {
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
-      const int r = (wm + 4 * m) * 16 + (lane & 15);
+      const int r = (wm + kGroupStep * m) * 16 + (lane & 15);
       if (r < ti.rows) as[m] = g.a_scale[ti.row0 + r];
     }
   }
@@ -330,12 +333,12 @@ __device__ __forceinline__ void epilogue(const GroupedGemmArgs& g, const TileInf
     }
   }
 #pragma unroll
-  for (int pass = 0; pass < 2; ++pass) {
+  for (int pass = 0; pass < (HALF ? 1 : 2); ++pass) {
     lds_barrier();  // the ring (or the last pass's rows) is no longer read
 #pragma unroll
-    for (int mm = 0; mm < 2; ++mm) {
-      const int m = 2 * pass + mm;
-      const int rl = (wm + 4 * mm) * 16 + (lane & 15);  // row within the pass
+    for (int mm = 0; mm < kPassGroups; ++mm) {
+      const int m = kPassGroups * pass + mm;
+      const int rl = (wm + kGroupStep * mm) * 16 + (lane & 15);  // row within the pass
       const float w = kWeighted && !OUT_F32 ? t_w[pass * 128 + rl] : 1.f;
       unsigned char* dst = lds + rl * kPitch + colw * kEsz;
 #pragma unroll
@@ -343,7 +346,7 @@ __device__ __forceinline__ void epilogue(const GroupedGemmArgs& g, const TileInf
         const f32x4_t a0 = acc[n][m] * sc0[n] * as[m];
         f32x4_t v;
         if constexpr (EPI == EPI_SWIGLU) {
-          const f32x4_t a1 = acc[n + 4][m] * sc1[n] * as[m];
+          const f32x4_t a1 = acc[n + kFrags][m] * sc1[n] * as[m];
           v = f32x4_t{silu_mul(a0[0], a1[0]), silu_mul(a0[1], a1[1]), silu_mul(a0[2], a1[2]), silu_mul(a0[3], a1[3])};
         } else {
           v = a0 * w;
@@ -394,6 +397,7 @@ struct WaveCtx {
   int a_lane;                  // LDS byte offset of this lane's A fragment in a 16-row group
   int wave, wm, wn;
   int KT;                      // stages of 32 inputs in this block's K range
+  bool only;                   // the expert's only row tile
 };
 
 // Fragment m of a wave covers 16-row group wm + 4 m of the tile, so the
@@ -562,17 +566,28 @@ __device__ __forceinline__ void k_body(const WaveCtx& c, f32x4_t (&acc)[8][4]) {
 // row set d & 1; d = 4, 5: weight blocks).
 // With two-term e4m3 activations (X2) the A halves are the stage's 64-input
 // piece of the hi codes (h = 0) and of the lo codes (h = 1).
-// HALF: tiles of at most 128 rows, whose stages hold 8 row groups (each wave
-// loads one) in a 5-deep ring; c.a_off[0] is then row group `wave`.
+// HALF: tiles of at most 128 rows.  Their stages hold 8 row groups (each wave
+// loads one; c.a_off[0] is row group `wave`) in a 5-deep ring, and the waves
+// are laid 2 x 4 instead of 4 x 2 over rows and columns: 16-row groups wm,
+// wm + 2, ... and 4 weight fragments a wave, so that a weight fragment is
+// converted by two waves instead of four.  The conversions bound these tiles:
+// at 83 rows a stage took 2100-2350 cycles, against some 1500 for its 16 KiB
+// from HBM and 770 for its MFMAs.  Measured (whole Mixtral block, full stages
+// -> 5 half stages -> and 2 x 4 waves -> and non-temporal loads): 333 tokens
+// 369 -> 363 -> 329 -> 327 us, 40 tokens 293 -> 263 -> 252 -> 252 us; two-term
+// activations, 300 tokens 391 -> 383 -> 362 -> 358 us.  Wider tiles stay 4 x 2:
+// their MFMAs cover the conversions and 2 x 4 reads more token rows from LDS.
 template <bool HALF>
 struct StageF8 {
   static constexpr int kAHalf = HALF ? kAStage / 2 : kAStage;  // one A half
   static constexpr int kBytes = 2 * kAHalf + kBStage;
   static constexpr int kRing = HALF ? 5 : kStagesF8;
   static constexpr int kLoads = HALF ? 4 : 6;                  // per wave
+  static constexpr int kFrags = HALF ? 4 : 8;                  // weight fragments per wave
+  static constexpr int kGroupStep = HALF ? 2 : 4;              // between a wave's token groups
 };
 
-template <bool X2, bool HALF>
+template <bool X2, bool HALF, bool NT>
 __device__ __forceinline__ void issue_one_f8(const WaveCtx& c, int kt, int buf, int d) {
   using S = StageF8<HALF>;
   constexpr int kALoads = S::kLoads - 2;
@@ -586,19 +601,25 @@ __device__ __forceinline__ void issue_one_f8(const WaveCtx& c, int kt, int buf, 
   } else {
     const int j = d - kALoads;
     unsigned char* dst = st + 2 * S::kAHalf + (c.wave * 2 + j) * 1024;
-    __builtin_amdgcn_global_load_lds(c.b_base[j] + (static_cast<uint32_t>(kt) * 1024 + c.b_lane), dst, 16, 0, 0);
+    const unsigned char* src = c.b_base[j] + (static_cast<uint32_t>(kt) * 1024 + c.b_lane);
+    if (NT)
+      __builtin_amdgcn_global_load_lds(src, dst, 16, 0, kNonTemporal);
+    else
+      __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
   }
 }
 
+template <bool HALF>
 __device__ __forceinline__ u32x4_t read_a_frag(const WaveCtx& c, const unsigned char* half_base, int m) {
-  return *reinterpret_cast<const u32x4_t*>(half_base + (c.wm + 4 * m) * 16 * 64 + c.a_lane);
+  return *reinterpret_cast<const u32x4_t*>(half_base + (c.wm + StageF8<HALF>::kGroupStep * m) * 16 * 64 + c.a_lane);
 }
 
 // Weight fragment n of a stage, still fp8: lane bytes 0-7 feed the first
 // 32-input half, bytes 8-15 the second.
-template <int NSETS>
+template <int NSETS, bool HALF>
 __device__ __forceinline__ u32x4_t read_b_frag(const WaveCtx& c, const unsigned char* b_base, int n) {
-  const int rb = NSETS == 2 ? ((n >> 2) * 8 + c.wn * 4 + (n & 3)) : (c.wn * 8 + n);
+  constexpr int kPerSet = StageF8<HALF>::kFrags / NSETS;
+  const int rb = (n / kPerSet) * 8 + c.wn * kPerSet + n % kPerSet;
   return *reinterpret_cast<const u32x4_t*>(b_base + rb * 1024 + c.b_lane);
 }
 
@@ -608,24 +629,24 @@ __device__ __forceinline__ u32x4_t convert_frag(const u32x4_t q) {
 }
 
 // This wave's loads of fp8 stage kt (its share) into buffer buf.
-template <bool X2, bool HALF>
+template <bool X2, bool HALF, bool NT>
 __device__ __forceinline__ void issue_share_f8(const WaveCtx& c, int kt, int buf) {
 #pragma unroll
-  for (int d = 0; d < StageF8<HALF>::kLoads; ++d) issue_one_f8<X2, HALF>(c, kt, buf, d);
+  for (int d = 0; d < StageF8<HALF>::kLoads; ++d) issue_one_f8<X2, HALF, NT>(c, kt, buf, d);
 }
 
 // A fragments of both 32-input halves and the 8 raw fp8 weight fragments of
 // the stage in buffer buf.
 template <int NM, int NSETS, bool HALF>
-__device__ __forceinline__ void read_stage_f8(const WaveCtx& c, int buf, u32x4_t (&fa)[2][4], u32x4_t (&fq)[8]) {
+__device__ __forceinline__ void read_stage_f8(const WaveCtx& c, int buf, u32x4_t (&fa)[2][4], u32x4_t (&fq)[StageF8<HALF>::kFrags]) {
   using S = StageF8<HALF>;
   const unsigned char* st = c.lds + buf * S::kBytes;
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int m = 0; m < NM; ++m) fa[h][m] = read_a_frag(c, st + h * S::kAHalf, m);
+    for (int m = 0; m < NM; ++m) fa[h][m] = read_a_frag<HALF>(c, st + h * S::kAHalf, m);
 #pragma unroll
-  for (int n = 0; n < 8; ++n) fq[n] = read_b_frag<NSETS>(c, st + 2 * S::kAHalf, n);
+  for (int n = 0; n < S::kFrags; ++n) fq[n] = read_b_frag<NSETS, HALF>(c, st + 2 * S::kAHalf, n);
 }
 
 // The 64 MFMAs of one fp8 stage, half by half; weight fragment n+1's codes
@@ -633,25 +654,25 @@ __device__ __forceinline__ void read_stage_f8(const WaveCtx& c, int buf, u32x4_t
 // activations (X2): one 16x16x128 fp8 MFMA per fragment pair, its first
 // operand the weight codes twice, its second the hi and the lo codes, so
 // the 128 products are w * hi and w * lo over the stage's 64 inputs.
-template <int NM, bool X2>
-__device__ __forceinline__ void multiply_f8(f32x4_t (&acc)[8][4], const u32x4_t (&fa)[2][4], const u32x4_t (&fq)[8]) {
+template <int NM, bool X2, int NF>
+__device__ __forceinline__ void multiply_f8(f32x4_t (&acc)[8][4], const u32x4_t (&fa)[2][4], const u32x4_t (&fq)[NF]) {
   if constexpr (X2) {
 #pragma unroll
-    for (int n = 0; n < 8; ++n)
+    for (int n = 0; n < NF; ++n)
 #pragma unroll
       for (int m = 0; m < NM; ++m) acc[n][m] = mfma_f8x2(fq[n], fq[n], fa[0][m], fa[1][m], acc[n][m]);
   } else if constexpr (NM > 0) {
     u32x4_t cur = convert_frag<0>(fq[0]);
 #pragma unroll
-    for (int n = 0; n < 8; ++n) {
-      const u32x4_t nxt = n < 7 ? convert_frag<0>(fq[n + 1]) : convert_frag<1>(fq[0]);
+    for (int n = 0; n < NF; ++n) {
+      const u32x4_t nxt = n < NF - 1 ? convert_frag<0>(fq[n + 1]) : convert_frag<1>(fq[0]);
 #pragma unroll
       for (int m = 0; m < NM; ++m) acc[n][m] = mfma16(cur, fa[0][m], acc[n][m]);
       cur = nxt;
     }
 #pragma unroll
-    for (int n = 0; n < 8; ++n) {
-      const u32x4_t nxt = n < 7 ? convert_frag<1>(fq[n + 1]) : cur;
+    for (int n = 0; n < NF; ++n) {
+      const u32x4_t nxt = n < NF - 1 ? convert_frag<1>(fq[n + 1]) : cur;
 #pragma unroll
       for (int m = 0; m < NM; ++m) acc[n][m] = mfma16(cur, fa[1][m], acc[n][m]);
       cur = nxt;
@@ -674,13 +695,13 @@ __device__ __forceinline__ void multiply_f8(f32x4_t (&acc)[8][4], const u32x4_t 
 // landing.  Loads past the last stage are not issued (those slots wait for
 // everything instead); the prologue re-reads the last stage into buffers
 // that are never read when K has fewer stages than the ring.
-template <int NM, int NSETS, int G, bool X2, bool HALF>
+template <int NM, int NSETS, int G, bool X2, bool HALF, bool NT>
 __device__ __forceinline__ void k_loop_f8(const WaveCtx& c, f32x4_t (&acc)[8][4]) {
   constexpr int R = StageF8<HALF>::kRing, kLoads = StageF8<HALF>::kLoads;
   const int KT = c.KT;
-  u32x4_t fa[2][4], fq[8];
+  u32x4_t fa[2][4], fq[StageF8<HALF>::kFrags];
 #pragma unroll
-  for (int s = 0; s < (G == 0 ? R : R - 1); ++s) issue_share_f8<X2, HALF>(c, s < KT ? s : KT - 1, s);
+  for (int s = 0; s < (G == 0 ? R : R - 1); ++s) issue_share_f8<X2, HALF, NT>(c, s < KT ? s : KT - 1, s);
   __builtin_amdgcn_s_waitcnt(wait_vm(kLoads * (G == 0 ? R - 1 : R - 2), false));
   asm volatile("s_barrier" ::: "memory");
   if constexpr (G == 0) {
@@ -695,7 +716,7 @@ __device__ __forceinline__ void k_loop_f8(const WaveCtx& c, f32x4_t (&acc)[8][4]
     if constexpr (G == 0) {
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_setprio(1);
-      multiply_f8<NM, X2>(acc, fa, fq);
+      multiply_f8<NM, X2, StageF8<HALF>::kFrags>(acc, fa, fq);
       __builtin_amdgcn_s_setprio(0);
       __builtin_amdgcn_sched_barrier(0);
       asm volatile("s_barrier" ::: "memory");
@@ -703,7 +724,7 @@ __device__ __forceinline__ void k_loop_f8(const WaveCtx& c, f32x4_t (&acc)[8][4]
       if constexpr (NM > 0)
         if (kt + 1 < KT) read_stage_f8<NM, NSETS, HALF>(c, rd, fa, fq);
       if (kt + R < KT) {
-        issue_share_f8<X2, HALF>(c, kt + R, wr);
+        issue_share_f8<X2, HALF, NT>(c, kt + R, wr);
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(wait_vm(kLoads * (R - 2), true));
       } else {
@@ -715,7 +736,7 @@ __device__ __forceinline__ void k_loop_f8(const WaveCtx& c, f32x4_t (&acc)[8][4]
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (NM > 0) read_stage_f8<NM, NSETS, HALF>(c, rd, fa, fq);
       if (kt + R - 1 < KT) {
-        issue_share_f8<X2, HALF>(c, kt + R - 1, wr);
+        issue_share_f8<X2, HALF, NT>(c, kt + R - 1, wr);
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(wait_vm(kLoads * (R - 2), true));
       } else {
@@ -725,7 +746,7 @@ __device__ __forceinline__ void k_loop_f8(const WaveCtx& c, f32x4_t (&acc)[8][4]
       asm volatile("s_barrier" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_setprio(1);
-      multiply_f8<NM, X2>(acc, fa, fq);
+      multiply_f8<NM, X2, StageF8<HALF>::kFrags>(acc, fa, fq);
       __builtin_amdgcn_s_setprio(0);
       __builtin_amdgcn_sched_barrier(0);
       asm volatile("s_barrier" ::: "memory");
@@ -737,27 +758,28 @@ __device__ __forceinline__ void k_loop_f8(const WaveCtx& c, f32x4_t (&acc)[8][4]
 }
 
 // The fp8-weight K loop of a tile with `rows` rows: this wave's active 16-row
-// groups (wm, wm + 4, ... below ceil(rows / 16), at most MAXM) select the
-// specialisation.
-template <int MAXM, int NSETS, bool X2, bool HALF>
+// groups (wm, wm + 4, ... below ceil(rows / 16); HALF: wm, wm + 2, ...) select
+// the specialisation.
+template <int NSETS, bool X2, bool HALF, bool NT>
 __device__ __forceinline__ void run_k_f8(const WaveCtx& c, f32x4_t (&acc)[8][4], int rows) {
+  constexpr int kStep = StageF8<HALF>::kGroupStep;
   const int groups = (rows + 15) >> 4;
-  const int nm = groups > c.wm ? min(MAXM, (groups - c.wm + 3) >> 2) : 0;
+  const int nm = groups > c.wm ? min(4, (groups - c.wm + kStep - 1) / kStep) : 0;
   if (c.wave < 4) {
     switch (nm) {
-      case 4: if constexpr (MAXM == 4) k_loop_f8<4, NSETS, 0, X2, HALF>(c, acc); break;
-      case 3: if constexpr (MAXM == 4) k_loop_f8<3, NSETS, 0, X2, HALF>(c, acc); break;
-      case 2: k_loop_f8<2, NSETS, 0, X2, HALF>(c, acc); break;
-      case 1: k_loop_f8<1, NSETS, 0, X2, HALF>(c, acc); break;
-      default: k_loop_f8<0, NSETS, 0, X2, HALF>(c, acc); break;
+      case 4: k_loop_f8<4, NSETS, 0, X2, HALF, NT>(c, acc); break;
+      case 3: k_loop_f8<3, NSETS, 0, X2, HALF, NT>(c, acc); break;
+      case 2: k_loop_f8<2, NSETS, 0, X2, HALF, NT>(c, acc); break;
+      case 1: k_loop_f8<1, NSETS, 0, X2, HALF, NT>(c, acc); break;
+      default: k_loop_f8<0, NSETS, 0, X2, HALF, NT>(c, acc); break;
     }
   } else {
     switch (nm) {
-      case 4: if constexpr (MAXM == 4) k_loop_f8<4, NSETS, 1, X2, HALF>(c, acc); break;
-      case 3: if constexpr (MAXM == 4) k_loop_f8<3, NSETS, 1, X2, HALF>(c, acc); break;
-      case 2: k_loop_f8<2, NSETS, 1, X2, HALF>(c, acc); break;
-      case 1: k_loop_f8<1, NSETS, 1, X2, HALF>(c, acc); break;
-      default: k_loop_f8<0, NSETS, 1, X2, HALF>(c, acc); break;
+      case 4: k_loop_f8<4, NSETS, 1, X2, HALF, NT>(c, acc); break;
+      case 3: k_loop_f8<3, NSETS, 1, X2, HALF, NT>(c, acc); break;
+      case 2: k_loop_f8<2, NSETS, 1, X2, HALF, NT>(c, acc); break;
+      case 1: k_loop_f8<1, NSETS, 1, X2, HALF, NT>(c, acc); break;
+      default: k_loop_f8<0, NSETS, 1, X2, HALF, NT>(c, acc); break;
     }
   }
 }
@@ -831,60 +853,49 @@ __device__ __forceinline__ WaveCtx tile_ctx(const GroupedGemmArgs& g, const Tile
   c.wm = wave >> 1;  // 16-row groups wm, wm+4, wm+8, wm+12
   c.wn = wave & 1;   // weight rows of each set: wn half
   c.KT = KT;
+  c.only = g.offsets[ti.expert + 1] - g.offsets[ti.expert] == ti.rows;
   return c;
 }
 
-// ---- Narrow tiles (bf16 activations; at most 128 rows, with fp8 weights 64).
-// Such a tile is bound by how many weight bytes are in flight, not by its
-// MFMAs, so it runs its own loop: stages that hold only the token rows it has
-// (MG = 1: 64, MG = 2: 128) beside the 16 weight blocks, in as deep a ring as
-// the LDS holds (bf16 8 or 6 stages of 20 or 24 KiB; fp8 weights, 64 inputs a
-// stage, 6 of 24 KiB) with all but two of them in flight, against 2-3 stages
-// of the main loops.  A wave loads its share of the token groups and two
-// weight blocks; one barrier per stage (a buffer is refilled two stages after
-// its last read).  Measured (whole block, before -> with this loop and the
-// loads below): bf16 Mixtral 64 / 160 / 333 / 480 tokens 531 -> 478, 544 -> 505,
+// ---- Narrow tiles (bf16 x bf16, at most 128 rows).  Such a tile is bound by
+// how many weight bytes are in flight, not by its MFMAs, so it runs its own
+// loop: stages that hold only the token rows it has (MG = 1: 64, MG = 2: 128)
+// beside the 16 weight blocks, in as deep a ring as the LDS holds (8 or 6
+// stages of 20 or 24 KiB) with all but two of them in flight, against 2-3
+// stages of the main loop.  A wave loads its share of the token groups and
+// two weight blocks; one barrier per stage (a buffer is refilled two stages
+// after its last read).  Measured (whole block, before -> with this loop and
+// the loads below): Mixtral 64 / 160 / 333 / 480 tokens 531 -> 478, 544 -> 505,
 // 571 -> 538, 594 -> 580 us; Qwen3 500 / 2043 tokens 219 -> 204, 350 -> 335 us;
-// DeepSeek-V2-Lite 300 / 1100 tokens 234 -> 220, 269 -> 258 us; fp8 Mixtral 40 /
-// 120 / 200 tokens 293 -> 263, 308 -> 279, 341 -> 307 us.  fp8 weights with 65-128
-// rows are no gain here (Mixtral 333 tokens 356 -> 407 us: every wave converts
-// the same 8 fragments in step and nothing multiplies meanwhile); they keep
-// the ping-pong of k_loop_f8 with a 5-deep ring of smaller stages (two 8 KiB
-// halves of token rows instead of 16 KiB), 369 -> 366 us there, and Mixtral x2
-// 300 tokens 391 -> 383 us.
-// An expert's only row tile loads its weights non-temporally; a narrow last
-// tile behind full ones shares them in L2.  Measured (whole block, default ->
-// non-temporal): Mixtral 200 tokens 544 -> 511 us, DeepSeek-V2-Lite 300 tokens
-// 235 -> 221 us, Qwen3 500 and 2043 tokens 212 -> 208 and 336 -> 331 us; on thin
-// last tiles too, the gate projection at Mixtral's 250 rows per expert went
-// 418 -> 456 us, and the main loop's stages lose far more (Mixtral 4096 tokens
-// 2345 -> 2618 us).
+// DeepSeek-V2-Lite 300 / 1100 tokens 234 -> 220, 269 -> 258 us.  fp8 weights gain
+// nothing from it over their own loop: at Mixtral 333 tokens it took 407 us
+// against 356 (the waves convert in step and nothing multiplies meanwhile).
+// An expert's only row tile loads its weights non-temporally (fp8 weights
+// likewise); a narrow last tile behind full ones shares them in L2.  Measured
+// (whole block, default -> non-temporal): Mixtral 200 tokens 544 -> 511 us,
+// DeepSeek-V2-Lite 300 tokens 235 -> 221 us, Qwen3 500 and 2043 tokens 212 -> 208
+// and 336 -> 331 us, Mixtral fp8 400 tokens 348 -> 344 us, with two-term
+// activations 100 tokens 304 -> 286 us; on thin last tiles too, the gate
+// projection at Mixtral's 250 rows per expert went 418 -> 456 us, and the main
+// loop's stages lose far more (Mixtral 4096 tokens 2345 -> 2618 us).
 constexpr int kNarrowRows = 128;
-constexpr int kNarrowRowsF8 = 64;
 
-template <int MG, bool F8>
+template <int MG>
 struct Narrow {
-  static constexpr int kHalves = F8 ? 2 : 1;               // 32-input halves of a stage
-  static constexpr int kHalfB = MG * 4 * 1024;
-  static constexpr int kABytes = kHalves * kHalfB;
+  static constexpr int kABytes = MG * 4 * 1024;
   static constexpr int kStageB = kABytes + kBStage;
   static constexpr int kRingN = kLds / kStageB;
   static constexpr int kAhead = kRingN - 2;                // stages in flight
-  static constexpr int kLoads = 3;                         // per wave; 2 of waves 4-7 with 4 token groups
-  static_assert(MG * kHalves <= 2, "one token group per wave");
 };
 
 // a_off: this wave's token group (wave % (4 MG)) in stage 0.
-template <int MG, bool F8, bool NT>
+template <int MG, bool NT>
 __device__ __forceinline__ void narrow_issue(const WaveCtx& c, uint32_t a_off, int kt, int buf) {
-  using W = Narrow<MG, F8>;
+  using W = Narrow<MG>;
   unsigned char* st = c.lds + buf * W::kStageB;
-  // fp8 with 4 groups: waves 0-3 load half 0, waves 4-7 half 1
-  const int half = F8 ? c.wave >> 2 : 0;
-  const uint32_t piece = static_cast<uint32_t>(F8 ? 2 * kt + half : kt);
-  unsigned char* a_dst = st + half * W::kHalfB + (MG == 1 ? c.wave & 3 : c.wave) * 1024;
-  const unsigned char* a_src = c.a_base + (a_off + piece * c.a_kstride);
-  if (F8 || MG == 2 || c.wave < 4) __builtin_amdgcn_global_load_lds(a_src, a_dst, 16, 0, 0);
+  unsigned char* a_dst = st + (MG == 1 ? c.wave & 3 : c.wave) * 1024;
+  const unsigned char* a_src = c.a_base + (a_off + static_cast<uint32_t>(kt) * c.a_kstride);
+  if (MG == 2 || c.wave < 4) __builtin_amdgcn_global_load_lds(a_src, a_dst, 16, 0, 0);
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const unsigned char* src = c.b_base[j] + (static_cast<uint32_t>(kt) * 1024 + c.b_lane);
@@ -896,20 +907,20 @@ __device__ __forceinline__ void narrow_issue(const WaveCtx& c, uint32_t a_off, i
   }
 }
 
-template <int NSETS, int MG, bool F8, bool NT>
+template <int NSETS, int MG, bool NT>
 __device__ __forceinline__ void narrow_k_loop(const WaveCtx& c, uint32_t a_off, int rows, f32x4_t (&acc)[8][4]) {
-  using W = Narrow<MG, F8>;
+  using W = Narrow<MG>;
   const int KT = c.KT;
   // this wave pair's row groups wm (and wm + 4) that hold rows
   const bool active0 = c.wm * 16 < rows, active1 = MG == 2 && (c.wm + 4) * 16 < rows;
-  for (int kt = 0; kt < W::kAhead && kt < KT; ++kt) narrow_issue<MG, F8, NT>(c, a_off, kt, kt);
+  for (int kt = 0; kt < W::kAhead && kt < KT; ++kt) narrow_issue<MG, NT>(c, a_off, kt, kt);
   for (int kt = 0; kt < KT; ++kt) {
     // Refill the buffer read two stages ago, then wait for stage kt (and for
     // this wave's reads of stage kt - 1, whose buffer the next trip refills).
     if (kt + W::kAhead < KT) {
-      narrow_issue<MG, F8, NT>(c, a_off, kt + W::kAhead, (kt + W::kAhead) % W::kRingN);
-      if (F8 || MG == 2 || c.wave < 4)
-        __builtin_amdgcn_s_waitcnt(wait_vm(W::kLoads * W::kAhead, true));
+      narrow_issue<MG, NT>(c, a_off, kt + W::kAhead, (kt + W::kAhead) % W::kRingN);
+      if (MG == 2 || c.wave < 4)
+        __builtin_amdgcn_s_waitcnt(wait_vm(3 * W::kAhead, true));
       else
         __builtin_amdgcn_s_waitcnt(wait_vm(2 * W::kAhead, true));
     } else {
@@ -918,12 +929,10 @@ __device__ __forceinline__ void narrow_k_loop(const WaveCtx& c, uint32_t a_off, 
     asm volatile("s_barrier" ::: "memory");
     if (active0) {
       const unsigned char* st = c.lds + (kt % W::kRingN) * W::kStageB;
-      u32x4_t fa[2][2], fb[8];
+      u32x4_t fa[MG], fb[8];
 #pragma unroll
-      for (int h = 0; h < W::kHalves; ++h)
-#pragma unroll
-        for (int m = 0; m < MG; ++m)
-          fa[h][m] = *reinterpret_cast<const u32x4_t*>(st + h * W::kHalfB + (c.wm + 4 * m) * 1024 + c.a_lane);
+      for (int m = 0; m < MG; ++m)
+        fa[m] = *reinterpret_cast<const u32x4_t*>(st + (c.wm + 4 * m) * 1024 + c.a_lane);
 #pragma unroll
       for (int n = 0; n < 8; ++n) {
         const int rb = NSETS == 2 ? ((n >> 2) * 8 + c.wn * 4 + (n & 3)) : (c.wn * 8 + n);
@@ -931,14 +940,8 @@ __device__ __forceinline__ void narrow_k_loop(const WaveCtx& c, uint32_t a_off, 
       }
 #pragma unroll
       for (int n = 0; n < 8; ++n) {
-        const u32x4_t w0 = F8 ? convert_frag<0>(fb[n]) : fb[n];
-        const u32x4_t w1 = F8 ? convert_frag<1>(fb[n]) : fb[n];
-        acc[n][0] = mfma16(w0, fa[0][0], acc[n][0]);
-        if (F8) acc[n][0] = mfma16(w1, fa[1][0], acc[n][0]);
-        if (MG == 2 && active1) {
-          acc[n][1] = mfma16(w0, fa[0][MG - 1], acc[n][1]);
-          if (F8) acc[n][1] = mfma16(w1, fa[1][MG - 1], acc[n][1]);
-        }
+        acc[n][0] = mfma16(fb[n], fa[0], acc[n][0]);
+        if (MG == 2 && active1) acc[n][1] = mfma16(fb[n], fa[MG - 1], acc[n][1]);
       }
     }
   }
@@ -946,22 +949,20 @@ __device__ __forceinline__ void narrow_k_loop(const WaveCtx& c, uint32_t a_off, 
 }
 
 // The narrow loop of tile ti whose A piece 0 is kb_first.
-template <int NSETS, bool F8>
+template <int NSETS>
 __device__ __forceinline__ void run_narrow(const GroupedGemmArgs& g, const TileInfo& ti, const WaveCtx& c, int lane,
                                            int64_t kb_first, f32x4_t (&acc)[8][4]) {
-  const bool only = g.offsets[ti.expert + 1] - g.offsets[ti.expert] == ti.rows;  // the expert's only row tile
+  const uint32_t a_off = a_group_offset(g, ti, ti.rows <= 64 ? c.wave & 3 : c.wave, lane, kb_first);
   if (ti.rows <= 64) {
-    const uint32_t a_off = a_group_offset(g, ti, c.wave & 3, lane, kb_first);
-    if (only)
-      narrow_k_loop<NSETS, 1, F8, true>(c, a_off, ti.rows, acc);
+    if (c.only)
+      narrow_k_loop<NSETS, 1, true>(c, a_off, ti.rows, acc);
     else
-      narrow_k_loop<NSETS, 1, F8, false>(c, a_off, ti.rows, acc);
-  } else if constexpr (!F8) {
-    const uint32_t a_off = a_group_offset(g, ti, c.wave, lane, kb_first);
-    if (only)
-      narrow_k_loop<NSETS, 2, F8, true>(c, a_off, ti.rows, acc);
+      narrow_k_loop<NSETS, 1, false>(c, a_off, ti.rows, acc);
+  } else {
+    if (c.only)
+      narrow_k_loop<NSETS, 2, true>(c, a_off, ti.rows, acc);
     else
-      narrow_k_loop<NSETS, 2, F8, false>(c, a_off, ti.rows, acc);
+      narrow_k_loop<NSETS, 2, false>(c, a_off, ti.rows, acc);
   }
 }
 
@@ -990,6 +991,17 @@ __device__ __forceinline__ void run_k_body(const WaveCtx& c, f32x4_t (&acc)[8][4
       default: k_body<0, NSETS, 1, A8>(c, acc); break;
     }
   }
+}
+
+template <int EPI, int NSETS, bool F8, bool A8, bool HALF>
+__device__ __forceinline__ void store_tile(const GroupedGemmArgs& g, const TileInfo& ti, int split, int64_t n0,
+                                            const WaveCtx& c, int lane, const f32x4_t (&acc)[8][4], const EpiRows& er) {
+  if constexpr (EPI == EPI_SWIGLU)
+    epilogue<EPI, NSETS, F8, A8, false, HALF>(g, ti, split, n0, c.wm, c.wn, lane, c.lds, acc, er);
+  else if (g.out_dtype == DT_F32)
+    epilogue<EPI, NSETS, F8, A8, true, HALF>(g, ti, split, n0, c.wm, c.wn, lane, c.lds, acc, er);
+  else
+    epilogue<EPI, NSETS, F8, A8, false, HALF>(g, ti, split, n0, c.wm, c.wn, lane, c.lds, acc, er);
 }
 
 // F8: e4m3 weights.  A8 (with F8): e4m3 activations too, K-blocked in
@@ -1050,34 +1062,36 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiled256_kernel(GroupedGemmA
 
   EpiRows er;
   epi_rows_first<EPI>(g, ti, er);
-  if (!A8 && ti.rows <= (F8 ? kNarrowRowsF8 : kNarrowRows)) {
-    // first 32-input A piece of this block's K range
-    const int kblocks = static_cast<int>(g.K / (F8 ? 64 : 32));
-    const int64_t kb_first = static_cast<int64_t>(split_boundary(kblocks, g.ksplit, split, g.ksplit_first64)) * (F8 ? 2 : 1);
-    run_narrow<NSETS, F8>(g, ti, c, lane, kb_first, acc);
-  } else if constexpr (F8 && (!A8 || X2)) {
+  if constexpr (F8 && (!A8 || X2)) {
     if (ti.rows <= kNarrowRows) {
       // A pieces of the K range's first stage: two 32-input bf16 pieces a
       // stage, or one 64-input piece of each term
-      const int k_first = split_boundary(static_cast<int>(g.K / 64), g.ksplit, split, g.ksplit_first64);
+      const int64_t kb_first =
+          static_cast<int64_t>(split_boundary(static_cast<int>(g.K / 64), g.ksplit, split, g.ksplit_first64)) *
+          (X2 ? 1 : 2);
       WaveCtx h = c;
-      h.a_off[0] = a_group_offset(g, ti, wave, lane, static_cast<int64_t>(k_first) * (X2 ? 1 : 2));
-      run_k_f8<2, NSETS, X2, true>(h, acc, ti.rows);
-    } else {
-      run_k_f8<4, NSETS, X2, false>(c, acc, ti.rows);
+      h.wm = (wave ^ (wave >> 2)) & 1;  // the two waves of a SIMD hold one half of the token groups each
+      h.wn = wave >> 1;
+      h.a_off[0] = a_group_offset(g, ti, wave, lane, kb_first);
+      if (c.only)
+        run_k_f8<NSETS, X2, true, true>(h, acc, ti.rows);
+      else
+        run_k_f8<NSETS, X2, true, false>(h, acc, ti.rows);
+      epi_rows_second<EPI>(g, ti, er);
+      store_tile<EPI, NSETS, F8, A8, true>(g, ti, split, n0, h, lane, acc, er);
+      return;
     }
+    run_k_f8<NSETS, X2, false, false>(c, acc, ti.rows);
+  } else if (!A8 && ti.rows <= kNarrowRows) {
+    // first 32-input A piece of this block's K range
+    const int64_t kb_first = split_boundary(static_cast<int>(g.K / 32), g.ksplit, split, g.ksplit_first64);
+    run_narrow<NSETS>(g, ti, c, lane, kb_first, acc);
   } else {
     k_issue_range<NSETS>(c, 0, 4);
     run_k_body<NSETS, A8>(c, acc, ti.rows);
   }
   epi_rows_second<EPI>(g, ti, er);
-
-  if constexpr (EPI == EPI_SWIGLU)
-    epilogue<EPI, NSETS, F8, A8, false>(g, ti, split, n0, c.wm, c.wn, lane, lds, acc, er);
-  else if (g.out_dtype == DT_F32)
-    epilogue<EPI, NSETS, F8, A8, true>(g, ti, split, n0, c.wm, c.wn, lane, lds, acc, er);
-  else
-    epilogue<EPI, NSETS, F8, A8, false>(g, ti, split, n0, c.wm, c.wn, lane, lds, acc, er);
+  store_tile<EPI, NSETS, F8, A8, false>(g, ti, split, n0, c, lane, acc, er);
 }
 
 template <int EPI, int NSETS, bool F8, bool A8, bool X2 = false>

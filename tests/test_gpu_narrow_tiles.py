@@ -1,5 +1,5 @@
 """Row tiles of at most 128 rows of the prefill GEMM (gemm_tiled256.hip:
-narrow_k_loop; k_loop_f8's stages of 128 rows) against the float64 oracle's
+narrow_k_loop; k_loop_f8's half stages and 2 x 4 waves) against the float64 oracle's
 grouped products, every expert holding a chosen number of rows."""
 
 from __future__ import annotations

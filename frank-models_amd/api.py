@@ -345,45 +345,48 @@ def permute(ids, n_expert: int):
 
 
 # ---------------------------------------------------------------- mul_mat_id
-_check_streams = {}  # device index -> the stream that reads id checks back
-_check_lock = threading.Lock()
 # Weight bytes a product may read from which its ids are checked apart from it
-# (_IdCheck): the check's own launch costs the host about 10 us, waiting for the
-# product costs its whole time (toy sizes 61 against 48 us a call, 35 MB of
-# weights 59.5 against 57; DeepSeek-V2-Lite's up projection, 8 tokens, 260 MB: 63
-# against 78 us; 96 tokens 93 against 119).
+# (_IdCheck): the check's launches cost 4-5 us of the stream, waiting for the
+# product costs the host its whole time.  Measured, apart against waiting, a call among
+# others and one whose result is waited for: toy sizes 44 / 55 against 48 / 51
+# us; DeepSeek-V2-Lite's up projection, 8 tokens (260 MB), 48 / 82 against 76 /
+# 79, 96 tokens 88 / 122 against 116 / 119.
 _CHECK_APART_BYTES = 128 << 20
+# Permutation workspace (the error word and, above 2048 ids, chunk histograms)
+# that _IdCheck keeps in host memory; about 30000 ids of 128 experts.
+_CHECK_HOST_BYTES = 8 << 10
 
 
 class _IdCheck:
     """Counts the ids outside [0, n_expert) on the current stream (fmoe_permute's
-    error word), to be read back once the calls that use them are launched: the
-    wait is for the count alone, on a stream of its own, so the host does not
-    wait for the product behind it."""
+    error word) into pinned host memory, to be read once the product is
+    launched: the host waits for the event behind the count, not for the
+    product, and no other stream is involved.  The permutation's kernels have
+    their workspace in that host memory while it is small, which saves the copy
+    behind them (DeepSeek-V2-Lite's up projection, 96 tokens, 93 -> 88 us a call
+    among others; 128 experts of 2048 x 768, 8000 ids, 147 -> 141 us)."""
 
     def __init__(self, ids, n_expert):
         k, T = (int(s) for s in ids.shape)
         self.n_expert = n_expert
         need = L.lib().fmoe_permute_workspace_bytes(k, T, n_expert)
-        need = (int(need) + 255) // 256 * 256
-        # the workspace, then order [k * T] and offsets [n_expert + 1]
-        self.ws = torch.empty(need + 4 * (k * T + n_expert + 1), dtype=torch.uint8, device=ids.device)
-        base = self.ws.data_ptr()
-        L.call("fmoe_permute", _ptr(ids), k, T, n_expert, base + need, base + need + 4 * k * T, base, need, _stream())
+        on_host = need <= _CHECK_HOST_BYTES
+        self.host = torch.empty(need if on_host else 4, dtype=torch.uint8, pin_memory=True)
+        self.count = ctypes.c_int32.from_address(self.host.data_ptr())
+        self.count.value = -1
+        # order [k * T] and offsets [n_expert + 1]
+        out = torch.empty(k * T + n_expert + 1, dtype=torch.int32, device=ids.device)
+        ws = self.host if on_host else torch.empty(need, dtype=torch.uint8, device=ids.device)
+        L.call("fmoe_permute", _ptr(ids), k, T, n_expert, _ptr(out), _ptr(out) + 4 * k * T, _ptr(ws), need, _stream())
+        if not on_host:
+            self.host.copy_(ws[:4], non_blocking=True)
         self.done = torch.cuda.Event()
         self.done.record()
 
     def raise_if_bad(self):
-        dev = self.ws.device
-        with _check_lock:
-            side = _check_streams.get(dev.index)
-            if side is None:
-                side = _check_streams[dev.index] = torch.cuda.Stream(dev)
-        side.wait_event(self.done)
-        bad = ctypes.c_int64(0)
-        L.call("fmoe_workspace_error_count", self.ws.data_ptr(), side.cuda_stream, ctypes.byref(bad))
-        if bad.value:
-            raise IndexError(f"ids: {bad.value} expert id(s) outside [0, {self.n_expert})")
+        self.done.synchronize()
+        if self.count.value:
+            raise IndexError(f"ids: {self.count.value} expert id(s) outside [0, {self.n_expert})")
 
 
 def mul_mat_id(weights, input, ids):
@@ -419,13 +422,18 @@ def mul_mat_id(weights, input, ids):
     k, T = (int(s) for s in d_ids.shape)
     if tuple(x.shape) != (n_in, k, T):
         raise ValueError(f"input shape {tuple(x.shape)} != {(n_in, k, T)}")
+    out = torch.empty((n_out, k, T), dtype=x.dtype, device=x.device)
+    ws = _workspace(L.lib().fmoe_mul_mat_id_workspace_bytes(n_out, n_in, n_expert, k, T, act))
     check = None
     if not checked and min(n_expert, k * T) * (pw.data.numel() // n_expert) > _CHECK_APART_BYTES:
         check = _IdCheck(d_ids, n_expert)
-    out = torch.empty((n_out, k, T), dtype=x.dtype, device=x.device)
-    ws = _workspace(L.lib().fmoe_mul_mat_id_workspace_bytes(n_out, n_in, n_expert, k, T, act))
-    L.call("fmoe_mul_mat_id", _ptr(pw.data), _ptr(pw.scales), pw.dtype, _ptr(x), _ptr(d_ids),
-           _ptr(out), n_out, n_in, n_expert, k, T, act, _ptr(ws), ws.numel(), _stream())
+    try:
+        L.call("fmoe_mul_mat_id", _ptr(pw.data), _ptr(pw.scales), pw.dtype, _ptr(x), _ptr(d_ids),
+               _ptr(out), n_out, n_in, n_expert, k, T, act, _ptr(ws), ws.numel(), _stream())
+    except Exception:
+        if check is not None:
+            check.done.synchronize()  # the host word stays until the device has written it
+        raise
     if check is not None:
         check.raise_if_bad()
     elif not checked and k * T > 0:

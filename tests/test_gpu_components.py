@@ -3,6 +3,10 @@ bit-exact), permutation (bit-exact), SwiGLU, packing (bf16 / fp8 bits),
 and the reference's own mul_mat_id / moe_ffn_block test cases at the
 reference's tolerance (rtol 1e-4, atol 1e-5)."""
 
+import importlib
+import threading
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -408,12 +412,19 @@ def test_row_quantizer_codes_match_the_oracle(fm, two_terms):
         assert not lo.any()
 
 
-@pytest.mark.parametrize("T", [8, 700])
-def test_mul_mat_id_device_ids_checked_apart(fm, T):
-    """Weights large enough that the ids are checked on a launch and a stream of
-    their own: out-of-range device ids still raise at the call, on the default
+@pytest.mark.parametrize("T,host_bytes", [(8, None), (700, None), (700, 0)])
+def test_mul_mat_id_device_ids_checked_apart(fm, monkeypatch, T, host_bytes):
+    """Weights large enough that the ids are checked apart from the product
+    (_IdCheck): out-of-range device ids still raise at the call, on the default
     and on another stream, and the calls around it are unaffected.  T = 700
-    with 4 slots: above the one-block permutation's 2048 ids."""
+    with 4 slots: above the one-block permutation's 2048 ids, its workspace in
+    host memory and, as for far larger calls, on the device."""
+    api = importlib.import_module("frank-models_amd.api")
+    if host_bytes is not None:
+        monkeypatch.setattr(api, "_CHECK_HOST_BYTES", host_bytes)
+    checks = []
+    read_back = api._IdCheck.raise_if_bad
+    monkeypatch.setattr(api._IdCheck, "raise_if_bad", lambda self: (checks.append(self.count), read_back(self)))
     n, E, k = 2048, 32, 4  # 256 MB of bf16 weights, every expert routed to
     g = torch.Generator(device="cuda").manual_seed(3)
     w = fm.pack_expert_weights(torch.randn((n, n, E), device="cuda", generator=g).bfloat16())
@@ -431,3 +442,76 @@ def test_mul_mat_id_device_ids_checked_apart(fm, T):
             again = fm.mul_mat_id(w, x, ids)
         torch.cuda.synchronize()
         assert torch.equal(good, again)
+    assert len(checks) == 7  # every call took this path
+
+
+def _stream_beside_the_current_one():
+    """A stream whose kernels run beside the current stream's (streams share a
+    few hardware queues), or None."""
+    tiny = torch.zeros(1, device="cuda")
+    for _ in range(8):
+        side = torch.cuda.Stream()
+        done = torch.cuda.Event()
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(_cycles(20.0))
+            done.record()
+        tiny.add_(1)
+        torch.cuda.current_stream().synchronize()
+        beside = not done.query()
+        torch.cuda.synchronize()
+        if beside:
+            return side
+    return None
+
+
+def _cycles(ms):
+    """torch.cuda._sleep's argument for about `ms` milliseconds."""
+    start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    start.record()
+    torch.cuda._sleep(1_000_000)
+    end.record()
+    torch.cuda.synchronize()
+    return int(1_000_000 * ms / start.elapsed_time(end))
+
+
+def test_mul_mat_id_waits_for_its_own_ids_only(fm, monkeypatch):
+    """The id check of a call on an idle stream does not wait for another
+    thread's call, whose stream still has a long queue before it."""
+    api = importlib.import_module("frank-models_amd.api")
+    monkeypatch.setattr(api, "_CHECK_APART_BYTES", -1)
+    n, E, k, T = 256, 8, 2, 16
+    g = torch.Generator(device="cuda").manual_seed(4)
+    w = fm.pack_expert_weights(torch.randn((n, n, E), device="cuda", generator=g).bfloat16())
+    x = torch.randn((n, k, T), device="cuda", generator=g).bfloat16()
+    ids = torch.rand((T, E), device="cuda", generator=g).topk(k, dim=1).indices.T.to(torch.int32).contiguous()
+    good = fm.mul_mat_id(w, x, ids)
+    busy = _stream_beside_the_current_one()
+    if busy is None:
+        pytest.skip("no stream runs beside the current one")
+    cycles = _cycles(500.0)
+    waiting, queue_done, results = threading.Event(), torch.cuda.Event(), []
+    read_back = api._IdCheck.raise_if_bad
+
+    def announced(self):
+        if threading.current_thread() is not threading.main_thread():
+            waiting.set()
+        read_back(self)
+
+    monkeypatch.setattr(api._IdCheck, "raise_if_bad", announced)
+
+    def other_thread():
+        with torch.cuda.stream(busy):
+            torch.cuda._sleep(cycles)
+            queue_done.record()
+            results.append(fm.mul_mat_id(w, x, ids))
+
+    thread = threading.Thread(target=other_thread)
+    thread.start()
+    assert waiting.wait(timeout=60)
+    time.sleep(0.05)  # the other thread is inside its wait
+    mine = fm.mul_mat_id(w, x, ids)
+    other_queue_ran_on = not queue_done.query()
+    thread.join()
+    torch.cuda.synchronize()
+    assert other_queue_ran_on
+    assert torch.equal(mine, good) and torch.equal(results[0], good)

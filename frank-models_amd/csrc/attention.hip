@@ -477,6 +477,11 @@ struct Ring {
   static_assert(kWaveB >= 2 * G * D * 4, "a wave's two partial outputs fit its ring");
 };
 
+// What the exponents of a chunk are taken against: its maximum, or 0 where every
+// score so far is minus infinity (finite keys whose products overflow, as
+// masking ones do), so that such positions weigh 0 and not NaN.
+__device__ __forceinline__ float finite_base(float m) { return m == -INFINITY ? 0.f : m; }
+
 // Non-temporal: a step reads each K and V byte once (with the default policy
 // the kernel takes 55.5 us at 16 x 4096 positions and 44.9 at 61 x 750).
 __device__ __forceinline__ void ring_load(const unsigned char* src, unsigned char* dst) {
@@ -635,12 +640,13 @@ __global__ __launch_bounds__(kAttnThreads, (Ring<D, G>::kBlocks)) void attn_ring
       for (int i = 0; i < 4; ++i) m = fmaxf(m, sc[it][i]);
     m = fmaxf(m, __shfl_xor(m, 16, kWave));
     m = fmaxf(m, __shfl_xor(m, 32, kWave));
+    const float base = finite_base(m);
     float sum = 0.f;
 #pragma unroll
     for (int it = 0; it < kT; ++it) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        sc[it][i] = __expf(sc[it][i] - m);
+        sc[it][i] = __expf(sc[it][i] - base);
         sum += sc[it][i];
       }
       if (col < G) *reinterpret_cast<f32x4_t*>(pw + col * kChunk + 16 * it + 4 * q4) = sc[it];
@@ -648,7 +654,7 @@ __global__ __launch_bounds__(kAttnThreads, (Ring<D, G>::kBlocks)) void attn_ring
     sum += __shfl_xor(sum, 16, kWave);
     sum += __shfl_xor(sum, 32, kWave);
     if (c > 0) {
-      const float f = __expf(m_old - m);
+      const float f = __expf(m_old - base);
       l = fmaf(l, f, sum);
 #pragma unroll
       for (int g = 0; g < G; ++g) {
@@ -738,11 +744,12 @@ __global__ __launch_bounds__(kAttnThreads, (Ring<D, G>::kBlocks)) void attn_ring
     float M = stat[g * 2];
 #pragma unroll
     for (int w = 1; w < kAttnWaves; ++w) M = fmaxf(M, stat[(w * G + g) * 2]);
+    const float base = finite_base(M);
     float o = 0.f, L = 0.f;
 #pragma unroll
     for (int w = 0; w < kAttnWaves; ++w) {
       const float* src = reinterpret_cast<const float*>(lds + w * R::kWaveB);
-      const float f = __expf(stat[(w * G + g) * 2] - M);  // 0 for a wave without positions
+      const float f = __expf(stat[(w * G + g) * 2] - base);  // 0 for a wave without positions
       o = fmaf(f, src[i] + src[G * D + i], o);
       L = fmaf(f, stat[(w * G + g) * 2 + 1], L);
     }

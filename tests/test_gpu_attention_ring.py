@@ -87,3 +87,32 @@ def test_ring_does_not_use_rows_past_the_context(fm):
     out, _, _ = blk.paged(x, lens[0].astype(np.int64), kp, vp, 0, tables, lens, 40, np.full(B, -1, np.int32),
                           np.zeros(B, np.int32))
     assert torch.isfinite(out).all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("masked", [(0, 64), (64, 128), (0, 256), (256, 300), (0, 300), (10, 290)])
+def test_ring_scores_of_minus_infinity(fm, D, masked):
+    """Cached keys of bf16's lowest value whose scores overflow to minus
+    infinity take no part, also where they fill a 64-position chunk of a wave,
+    a whole split, or the whole context."""
+    bs, ctx, q0 = 16, 300, 1000.0
+    rng = np.random.default_rng(D + masked[0])
+    w, zero = torch.zeros((D, D)), torch.zeros((D, D))
+    w[0, 0] = 1.0  # the query is x's first channel, the new token's key and value are zero
+    blk = fm.AttentionBlockDecode(*(m.cuda().bfloat16() for m in (w, zero, zero, torch.eye(D))), n_head=1, n_head_kv=1,
+                                  n_embd=D, act_dtype=torch.bfloat16)
+    x = torch.zeros((1, D))
+    x[0, 0] = q0
+    n_blocks = ctx // bs + 1
+    k = np.zeros((n_blocks * bs, D), np.float32)
+    v = nm.bf16_round(rng.standard_normal((n_blocks * bs, D)).astype(np.float32))
+    k[:, 0] = nm.bf16_round((rng.standard_normal(n_blocks * bs) * 1e-2).astype(np.float32))
+    k[masked[0]:masked[1], 0] = torch.finfo(torch.bfloat16).min
+    kd, vd = (torch.from_numpy(a).cuda().bfloat16().view(n_blocks, bs, 1, D) for a in (k, v))
+    out, _, _ = blk.paged(x.cuda().bfloat16(), np.zeros(1, np.int64), kd, vd, 0,
+                          np.arange(n_blocks, dtype=np.int32).reshape(1, 1, n_blocks), np.array([[ctx]], np.int32), ctx,
+                          np.full(1, -1, np.int32), np.zeros(1, np.int32))
+    keep = np.r_[0:masked[0], masked[1]:ctx]
+    score = np.append(q0 * D ** -0.5 * k[keep, 0].astype(np.float64), 0.0)  # the last: the new token's
+    p = np.exp(score - score.max())
+    assert_close_rms(out.float().cpu().numpy()[0], p[:-1] @ v[keep] / p.sum(), 1e-2)

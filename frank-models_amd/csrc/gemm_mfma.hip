@@ -26,7 +26,8 @@
 //           pass, 8 input steps of loads in flight per wave (16 for the
 //           one-tile bf16 gate/up kernel); one-weight projections stream
 //           through a ring in LDS instead (gemm_stream_lds_kernel up to 16
-//           rows, gemm_proj_kernel up to 128 and with fp8 weights).
+//           rows, gemm_proj_kernel beyond and with fp8 weights; the lines are
+//           at gemm_stream_fused_rows and proj_partial_round).
 //           For decode batches of at most 4 tokens the gate/up kernel can run
 //           the router's top-k and grouping in its own blocks (RoutePrologue),
 //           one launch fewer.
@@ -706,7 +707,8 @@ __global__ __launch_bounds__(kThreads + kRopeWaves * kWave) void gemm_stream_lds
 }
 
 // ============================================= projections of 17 to 128 rows
-// The same projections for more rows (and with fp8 weights): block = 16 * NB
+// The same projections for more rows (gemm_stream_fused_rows), and with fp8
+// weights (but proj_partial_round): block = 16 * NB
 // columns against all MT 16-row tiles, its 4 waves splitting the input axis in
 // units of 64 inputs.  Each wave streams its units through a ring of D slots
 // of its own in LDS (global_load_lds, no staging registers, no barrier in the
@@ -726,10 +728,12 @@ __global__ __launch_bounds__(kThreads + kRopeWaves * kWave) void gemm_stream_lds
 // launch) -> 20.5 us; output projection 24.4 us (gemm_stream_kernel) -> 13.2
 // us; whole step with 17 / 32 / 64 / 128 rows x 256 positions 57.0 / 62.6 /
 // 85.1 / 112 -> 47.8 / 51.3 / 60.3 / 102 us, and with fp8 weights at 16 / 32 /
-// 64 / 128 rows 46.8 / 62.1 / 77.1 / 105 -> 42.4 / 44.3 / 54.6 / 97.8 us.
+// 64 / 128 rows 46.8 / 62.1 / 77.1 / 105 -> 42.4 / 44.3 / 54.6 / 97.8 us.  (At 128
+// rows Q/K/V goes to the split product now: gemm_stream_fused_rows.)
 constexpr int kProjMaxRows = 128;
 constexpr int kProjWaves = 4;
 constexpr int kProjThreads = kProjWaves * kWave;
+constexpr int kProjRound = 256;  // resident blocks: one per CU
 
 template <int MT, int NB, bool F8>
 struct Proj {
@@ -1122,10 +1126,6 @@ void launch_stream_tiles(const GroupedGemmArgs& g, hipStream_t s, dim3 grid, int
   }
   if (g.epi == EPI_SWIGLU)
     hipLaunchKernelGGL((gemm_stream_kernel<EPI_SWIGLU, 2, F8, TILES>), grid, dim3(kThreads), 0, s, g, col_tiles);
-  else if (g.epi == EPI_LINEAR)
-    hipLaunchKernelGGL((gemm_stream_kernel<EPI_LINEAR, 1, F8, TILES>), grid, dim3(kThreads), 0, s, g, col_tiles);
-  else if (g.epi == EPI_QKV_ROPE)  // up to 16 rows (gemm_stream_fused_rows)
-    hipLaunchKernelGGL((gemm_stream_kernel<EPI_QKV_ROPE, 1, F8, 1>), grid, dim3(kThreads), 0, s, g, col_tiles);
   else if (g.epi == EPI_SCATTER_WEIGHTED)
     hipLaunchKernelGGL((gemm_stream_kernel<EPI_SCATTER_WEIGHTED, 1, F8, TILES>), grid, dim3(kThreads), 0, s, g,
                        col_tiles);
@@ -1225,12 +1225,32 @@ hipError_t launch_proj_n(const GroupedGemmArgs& g, hipStream_t s) {
 
 // Two column groups per block above 256 groups: a block then reads its token
 // rows for twice the columns and the grid is one round of one block per CU.
+int proj_col_groups(const GroupedGemmArgs& g) { return g.N > 16 * kProjRound && g.N % 32 == 0 ? 2 : 1; }
+
 template <int EPI, int MT, bool F8>
 hipError_t launch_proj_m(const GroupedGemmArgs& g, hipStream_t s) {
-  if (g.N > 16 * 256 && g.N % 32 == 0) {
-    if constexpr (MT <= 4) return launch_proj_n<EPI, MT, 2, F8>(g, s);
+  if constexpr (MT <= 4) {
+    if (proj_col_groups(g) == 2) return launch_proj_n<EPI, MT, 2, F8>(g, s);
   }
   return launch_proj_n<EPI, MT, 1, F8>(g, s);
+}
+
+// fp8 projections of at most kProjRegisterRows rows whose gemm_proj_kernel grid
+// leaves a quarter or more of its last round empty: at so few rows the round
+// is the weight stream alone, and gemm_stream_kernel's smaller blocks share the
+// CUs evenly.  Measured (Q/K/V, gemm_proj_kernel against gemm_stream_kernel, 1 /
+// 8 / 12 / 16 rows): 8192 -> 10240 (320 blocks) 30.2 / 31.0 / 31.1 / 32.5 against
+// 21.9 / 26.0 / 30.0 / 33.9 us, 4096 -> 12288 (384) 18.2 / 18.4 / 18.9 / 19.3
+// against 13.8 / 15.6 / 17.4 / 19.9, 3072 -> 9216 (288) 14.1 / 14.3 / 14.9 / 15.3
+// against 11.4 / 13.0 / 14.4 / 16.0; 5120 -> 15360 (480, the last round nearly
+// full) 22.4 / 22.9 / 24.0 / 25.8 against 22.5 / 25.0 / 26.7 / 29.9.
+constexpr int kProjRegisterRows = 12;
+
+bool proj_partial_round(const GroupedGemmArgs& g) {
+  const int64_t per = 16 * proj_col_groups(g);
+  const int64_t blocks = (g.N + per - 1) / per;
+  const int64_t rounds = (blocks + kProjRound - 1) / kProjRound;
+  return rounds > 1 && 4 * blocks <= 3 * kProjRound * rounds;
 }
 
 template <int EPI, bool F8>
@@ -1278,8 +1298,26 @@ hipError_t launch_stream_t(const GroupedGemmArgs& g, hipStream_t s) {
                          dim3(stream_lds_threads<EPI_QKV_ROPE>()), (stream_lds_bytes<kDepth, EPI_QKV_ROPE>()), s, g);
     return hipGetLastError();
   }
-  if ((g.epi == EPI_LINEAR || g.epi == EPI_QKV_ROPE) && g.K % 64 == 0 && g.n_assign <= kProjMaxRows)
+  if (g.epi == EPI_LINEAR || g.epi == EPI_QKV_ROPE) {
+    if (g.n_assign > gemm_stream_fused_rows(g)) return hipErrorNotSupported;
+    if constexpr (F8) {
+      if (g.n_assign <= kProjRegisterRows && proj_partial_round(g)) {
+        if (g.epi == EPI_LINEAR)
+          hipLaunchKernelGGL((gemm_stream_kernel<EPI_LINEAR, 1, true, 1>), grid, dim3(kThreads), 0, s, g, col_tiles);
+        else
+          hipLaunchKernelGGL((gemm_stream_kernel<EPI_QKV_ROPE, 1, true, 1>), grid, dim3(kThreads), 0, s, g, col_tiles);
+        return hipGetLastError();
+      }
+    } else if (g.K % 64) {  // 17 to 64 rows, EPI_LINEAR
+      if (g.epi != EPI_LINEAR) return hipErrorNotSupported;
+      if (rows <= 32)
+        hipLaunchKernelGGL((gemm_stream_kernel<EPI_LINEAR, 1, false, 2>), grid, dim3(kThreads), 0, s, g, col_tiles);
+      else
+        hipLaunchKernelGGL((gemm_stream_kernel<EPI_LINEAR, 1, false, 4>), grid, dim3(kThreads), 0, s, g, col_tiles);
+      return hipGetLastError();
+    }
     return g.epi == EPI_LINEAR ? launch_proj<EPI_LINEAR, F8>(g, s) : launch_proj<EPI_QKV_ROPE, F8>(g, s);
+  }
   if (rows <= 16)
     launch_stream_tiles<F8, 1>(g, s, grid, col_tiles);
   else if (rows <= 32)
@@ -1309,13 +1347,28 @@ bool proj_epilogue_ok(const GroupedGemmArgs& g) {
          g.N == static_cast<int64_t>(e.nq) + 2 * e.nkv;
 }
 
-// gemm_proj_kernel's range where it runs (its comment has both sides); the
-// register kernel's otherwise: its RoPE epilogue's angles run on one wave per
-// block (Q/K/V at 64 rows 44.5 us against 38.6 with a launch of their own), its
-// output projection streams up to 64 rows (24.7 us, level with the split
-// product + launch).
+// Rows of a projection on gemm_proj_kernel (K a multiple of 64).  Above 64 rows
+// a block takes one column group, one block per CU, so its time grows with the
+// rounds of the grid times K, while the split tile product and its launch for
+// the bias or RoPE cost little more than at 64 rows.  Measured, gemm_proj_kernel
+// against the split product at 65 / 96 / 97 / 128 rows (in brackets rounds x K):
+//   bf16, Q/K/V 2048 -> 6144 (4096)     19.9 / 21.5 / 23.4 / 24.4 against 26.4 / 28.1 / 28.9 / 30.6 us
+//   bf16, Q/K/V 3072 -> 4608 (6144)     25.2 / 27.6 / 30.6 / 31.9 against - / - / 31.1 / 32.4
+//   bf16, Q/K/V 4096 -> 6144 (8192)     30.8 / 34.0 / 37.2 / 39.6 against - / - / 36.0 / 38.4
+//   bf16, Q/K/V 3072 -> 9216 (9216)     37.5 / 40.8 / 44.2 / 47.0 against 34.1 / 37.9 / 38.3 / 40.8
+//   bf16, Q/K/V 8192 -> 10240 (24576)   75.7 / 85.6 / 92.6 / 101 against 57.4 / 64.3 / 64.5 / 70.7
+//   fp8, Q/K/V 3072 -> 4608 (6144)      23.2 / 25.4 / 28.6 / 30.3 against 24.8 / 26.3 / 27.9 / 28.9
+//   fp8, Q/K/V 4096 -> 6144 (8192)      28.4 / 30.7 / 34.1 / 36.3 against 26.8 / 28.9 / 30.5 / 32.3
+//   fp8, Q/K/V 8192 -> 10240 (24576)    64.9 / 73.8 / 81.9 / 89.6 against 40.7 / 44.4 / 44.7 / 49.2
+// For other K the register kernel: a RoPE epilogue's angles would run on one
+// wave per block there (Q/K/V at 64 rows 44.5 us against 38.6 with a launch of
+// their own), its output projection streams up to 64 rows (24.7 us, level with
+// the split product + launch).
 int gemm_stream_fused_rows(const GroupedGemmArgs& g) {
-  return g.K % 64 == 0 ? kProjMaxRows : g.epi == EPI_LINEAR ? 64 : 16;
+  if (g.K % 64) return g.epi == EPI_LINEAR ? 64 : 16;
+  const int64_t cost = (g.N + 16 * kProjRound - 1) / (16 * kProjRound) * g.K;
+  const bool f8 = g.w_dtype == DT_F8;
+  return cost <= (f8 ? 4096 : 6144) ? kProjMaxRows : cost <= (f8 ? 6144 : 8192) ? 96 : 64;
 }
 
 bool gemm_stream_routed_ok(const GroupedGemmArgs& g) {

@@ -1,6 +1,7 @@
 """The decode attention's projections at 17 to 128 rows (gemm_proj_kernel:
 bias + RoPE, and bias + residual, in its epilogue), and with fp8 weights at
-any row count up to that, against the float64 oracle.
+any row count up to that, against the float64 oracle, on both sides of the
+lines to the split product and to the register kernel.
 
 Bounds.  v_new is one product: K exact bf16 products summed in fp32 in any
 order (at most K 2^-24 sum |x w|), then one rounding to bf16 (2^-8 |v|).  k_new
@@ -38,7 +39,10 @@ def _weights(rng, n_in, n_out, fp8):
 
 # B: both sides of each row-tile count; n_embd 64 and 192: fewer units than
 # waves, and a wave without any; 4160 columns of Q/K/V: two column groups per
-# block; head sizes below and above a column group.
+# block; head sizes below and above a column group.  The last two rows: both
+# sides of the row limits (96 and 64 rows of Q/K/V 4096 -> 6144, 96 and 128 of
+# 3072 -> 4608), and 9216 columns of Q/K/V at 12 and 13 rows with fp8 weights
+# (288 blocks of two column groups, a second round nearly empty).
 @pytest.mark.parametrize("B,n_embd,H,Hkv,fp8,bias", [
     (17, 64, 4, 2, False, True), (32, 192, 6, 6, False, False), (33, 2560, 40, 10, False, True),
     (48, 512, 4, 4, False, False), (49, 256, 16, 2, False, True), (64, 2560, 20, 20, False, True),
@@ -46,6 +50,8 @@ def _weights(rng, n_in, n_out, fp8):
     (128, 256, 8, 1, False, True), (129, 256, 8, 1, False, True),
     (1, 64, 4, 2, True, True), (16, 2560, 40, 10, True, False), (17, 192, 6, 6, True, True),
     (64, 2560, 20, 20, True, False), (100, 256, 2, 2, True, True),
+    (96, 4096, 32, 8, False, True), (97, 4096, 32, 8, False, True), (65, 4096, 32, 8, True, False),
+    (97, 3072, 24, 6, True, True), (12, 3072, 24, 24, True, True), (13, 3072, 24, 24, True, True),
 ])
 def test_projections(fm, B, n_embd, H, Hkv, fp8, bias):
     rng = np.random.default_rng(B * 31 + n_embd)

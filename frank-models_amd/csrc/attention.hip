@@ -213,6 +213,7 @@ struct AttnArgs {
   int n_head, n_head_kv;
   int n_split;
   int split_len;          // positions per split
+  bool split_major;       // attn_ring_kernel: every sequence's split s before any split s + 1
   float scale;
   float* part;            // [B, n_head, n_split, D + 2]: o[D], m, l
 };
@@ -222,8 +223,8 @@ constexpr int kAttnThreads = 256;  // one thread per position of a split (rows[]
 static_assert(kAttnThreads == kSplitLen, "the rows[] fill gives each thread one position");
 constexpr int kAttnWaves = kAttnThreads / kWave;
 
-// fp32 pools, head_dim 16 and 32, and bf16 pools that are not 16-byte aligned
-// (attn_ring_kernel below takes the others).
+// fp32 pools, and bf16 pools with head_dim 16 and 32 (attn_ring_kernel below
+// takes the others).
 // Block (split s of kSplitLen positions, KV head, sequence b); wave w owns the
 // split's positions [64 w, 64 w + 64) in both phases, so a wave's memory traffic is two
 // rounds of independent loads: all of its K rows, then (issued before the
@@ -430,10 +431,10 @@ __global__ __launch_bounds__(kAttnThreads) void attn_split_kernel(AttnArgs a) {
   }
 }
 
-// bf16 pools with head_dim 64 or 128 (16-byte aligned pools): the same block
+// bf16 pools with head_dim 64 or 128, 16-byte aligned: the same block
 // (split, KV head, sequence) and partial results, with no block barrier
-// between its loads.  A block's positions (split_len of them: 256, 512 or
-// 1024) go to its waves in chunks of 64, chunk i to wave i % 4.  A chunk is
+// between its loads.  A block's positions (split_len of them, 256 to 1024) go
+// to its W waves in chunks of 64, chunk i to wave i % W (ring_plan).  A chunk is
 // four 16-position tiles of K, then four of V, which pass through a ring of
 // kSlots tiles of the wave's own in LDS (global_load_lds): a slot is refilled
 // as soon as its tile has been used, so loads stay in flight through the
@@ -460,7 +461,7 @@ constexpr int kSlots = 4;
 constexpr int kChunk = 64;      // positions of a wave per round of the ring
 constexpr int kMaxSplitLen = 1024;
 
-template <int D, int G>
+template <int D, int G, int W>
 struct Ring {
   static constexpr int kRowB = D * 2;
   static constexpr int kRowsPerLoad = 1024 / kRowB;             // 4 or 8
@@ -470,9 +471,9 @@ struct Ring {
   static constexpr int kWaveB = kSlots * kTileB;
   static constexpr int kRowIds = kMaxSplitLen / kAttnWaves;     // per wave
   static constexpr int kP = kChunk * G;                         // probabilities per wave
-  static constexpr int kLds = kAttnWaves * (kWaveB + kRowIds * 4 + kP * 4 + G * 8);
-  // blocks per CU the registers must allow
-  static constexpr int kBlocks = (D == 64 ? 3 : 2) - (G == 8 ? 1 : 0);
+  static constexpr int kLds = W * (kWaveB + kRowIds * 4 + kP * 4 + G * 8);
+  // waves per SIMD the registers must allow: blocks of four waves per CU
+  static constexpr int kPerSimd = (D == 64 ? 3 : 2) - (G == 8 ? 1 : 0);
   static_assert(kSlots == kTiles, "K tile i and V tile i share slot i");
   static_assert(kWaveB >= 2 * G * D * 4, "a wave's two partial outputs fit its ring");
 };
@@ -488,18 +489,19 @@ __device__ __forceinline__ void ring_load(const unsigned char* src, unsigned cha
   __builtin_amdgcn_global_load_lds(src, dst, 16, 0, kNonTemporal);
 }
 
-template <int D, int G>
-__global__ __launch_bounds__(kAttnThreads, (Ring<D, G>::kBlocks)) void attn_ring_kernel(AttnArgs a) {
-  using R = Ring<D, G>;
+template <int D, int G, int W>
+__global__ __launch_bounds__(W * kWave, (Ring<D, G, W>::kPerSimd)) void attn_ring_kernel(AttnArgs a) {
+  using R = Ring<D, G, W>;
   constexpr int kL = R::kLoads, kT = R::kTiles, kChunks = R::kRowB / 16;
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
-  const int s = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
+  const int s = a.split_major ? blockIdx.z : blockIdx.x, kvh = a.split_major ? blockIdx.x : blockIdx.y;
+  const int b = a.split_major ? blockIdx.y : blockIdx.z;
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   unsigned char* ring = lds + wave * R::kWaveB;
-  int* rows = reinterpret_cast<int*>(lds + kAttnWaves * R::kWaveB) + wave * R::kRowIds;
-  float* pw = reinterpret_cast<float*>(lds + kAttnWaves * (R::kWaveB + R::kRowIds * 4)) + wave * R::kP;  // [G][64]
-  float* stat = reinterpret_cast<float*>(lds + kAttnWaves * (R::kWaveB + R::kRowIds * 4 + R::kP * 4));  // [waves][G][m, l]
+  int* rows = reinterpret_cast<int*>(lds + W * R::kWaveB) + wave * R::kRowIds;
+  float* pw = reinterpret_cast<float*>(lds + W * (R::kWaveB + R::kRowIds * 4)) + wave * R::kP;  // [G][64]
+  float* stat = reinterpret_cast<float*>(lds + W * (R::kWaveB + R::kRowIds * 4 + R::kP * 4));  // [waves][G][m, l]
 
   // Query operand: lane (g = l / 16, column l % 16) holds 8 dimensions at
   // chunk 4 ks + g of head l % 8, the high part in columns 0-7, the remainder
@@ -520,9 +522,9 @@ __global__ __launch_bounds__(kAttnThreads, (Ring<D, G>::kBlocks)) void attn_ring
   if (n_b <= j0) return;  // block-uniform; the combine reads only the splits with positions
   const int len = min(a.split_len, n_b - j0);
   const int n_all = (len + kChunk - 1) / kChunk;
-  const int n = n_all > wave ? (n_all - wave + kAttnWaves - 1) / kAttnWaves : 0;  // this wave's chunks
+  const int n = n_all > wave ? (n_all - wave + W - 1) / W : 0;  // this wave's chunks
   for (int c = 0; c < n; ++c) {
-    const int t = (c * kAttnWaves + wave) * kChunk + lane;
+    const int t = (c * W + wave) * kChunk + lane;
     const int j = j0 + t;
     const int lb = j / a.block_size;
     int r = -2;  // past the context
@@ -739,15 +741,15 @@ __global__ __launch_bounds__(kAttnThreads, (Ring<D, G>::kBlocks)) void attn_ring
   }
   __syncthreads();
   float* part = a.part + (static_cast<int64_t>(b) * a.n_head + kvh * G) * a.n_split * (D + 2);
-  for (int i = tid; i < G * D; i += kAttnThreads) {
+  for (int i = tid; i < G * D; i += W * kWave) {
     const int g = i / D, d = i - g * D;
     float M = stat[g * 2];
 #pragma unroll
-    for (int w = 1; w < kAttnWaves; ++w) M = fmaxf(M, stat[(w * G + g) * 2]);
+    for (int w = 1; w < W; ++w) M = fmaxf(M, stat[(w * G + g) * 2]);
     const float base = finite_base(M);
     float o = 0.f, L = 0.f;
 #pragma unroll
-    for (int w = 0; w < kAttnWaves; ++w) {
+    for (int w = 0; w < W; ++w) {
       const float* src = reinterpret_cast<const float*>(lds + w * R::kWaveB);
       const float f = __expf(stat[(w * G + g) * 2] - base);  // 0 for a wave without positions
       o = fmaf(f, src[i] + src[G * D + i], o);
@@ -771,7 +773,7 @@ __global__ __launch_bounds__(kAttnThreads, (Ring<D, G>::kBlocks)) void attn_ring
 constexpr int kCombineThreads = 128;  // >= head_dim
 constexpr int kCombineChunk = 1024;   // splits whose weights are held in LDS at once
 constexpr int kCombineUnroll = 16;
-constexpr int kCombinePre = 16;       // splits (4096 positions) prefetched into registers
+constexpr int kCombinePre = 16;       // splits (4096 to 16384 positions) prefetched into registers
 
 // Blocks x = n_head and n_head + 1 (launched only with a scatter) write
 // k_new / v_new into the pools: the split kernel has read them by then.
@@ -866,32 +868,100 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(AttnArgs 
 constexpr int kLanesPerPos64 = 8;
 constexpr int kLanesPerPos128 = 8;
 
-// Positions per split: the most that still gives the GPU two blocks per CU.
-// Longer splits spend fewer prologues and merges (whole step at 16 x 4096
-// positions: 94.3 us with 256, 92.7 with 512, 91.4 with 1024; 128 x 380: 126,
-// 122, 122).
-int ring_split_len(int max_ctx, int64_t heads) {
-  int len = kMaxSplitLen;
-  while (len > kSplitLen && heads * ((max_ctx + len - 1) / len) < 512) len /= 2;
-  return len;
+// How attn_ring_kernel covers `heads` (sequence, KV head) pairs of contexts up
+// to max_ctx.  Measured: time of the attention kernels, the split kernel of 256
+// positions (one block per 256 positions, whatever the batch) against the choice.
+struct RingPlan {
+  int split_len, waves;
+  bool split_major;
+};
+
+// Time of a launch in units of 256 positions of one block, of one unit of
+// overhead per block, where `round` blocks are resident and the full splits come
+// first.
+int64_t ring_rounds(int max_ctx, int64_t heads, int len, int round) {
+  const int64_t n = (max_ctx + len - 1) / len, full = heads * (n - 1);
+  const int64_t rounds = (full + round - 1) / round, idle = rounds * round - full;
+  const int64_t last = (max_ctx - (n - 1) * len + kSplitLen - 1) / kSplitLen + 1;
+  return rounds * (len / kSplitLen + 1) + (heads > idle ? (heads - idle + round - 1) / round * last : 0);
+}
+
+RingPlan ring_plan(int max_ctx, int64_t heads, int head_dim, int group) {
+  RingPlan p{kMaxSplitLen, kAttnWaves, false};
+  // head_dim 128 with 8 query heads keeps one wave per SIMD, the others two
+  const bool one = head_dim == 128 && group == 8;
+  const int round = one ? 256 : 512;
+  // Short contexts of many pairs: a block of four waves reserves LDS and SIMD
+  // slots for waves that have no chunk, so the blocks get fewer waves, each with
+  // a chunk (one wave per SIMD: with enough chunks to fill the SIMDs).  8 query
+  // heads x 128, pairs x positions: 1024 x 64 39.6 -> 28.4 us (four waves: 46.8),
+  // 1024 x 256 55.9 -> 44.5 (59.6), 512 x 256 33.4 -> 28.2 (33.1), 1024 x 512
+  // 85.4 -> 73.6 (83.1).  1 query head x 128: 2048 x 16 26.9 -> 19.6 (30.8), 4096 x
+  // 48 53.5 -> 34.9 (56.1), 4096 x 128 78.1 -> 61.1 (66.0); 4 query heads: 1024 x 64
+  // 28.3 -> 21.8 (24.3).  Up to one round of four-wave blocks they are level or
+  // ahead (256 pairs x 64: 13.1 us, with one wave 14.2).
+  if (heads > round) {
+    if (max_ctx <= kChunk || (one && max_ctx <= kSplitLen && heads >= 4 * round))
+      p.waves = 1;
+    else if (max_ctx <= (one ? 2 * kSplitLen : 2 * kChunk))
+      p.waves = 2;
+    if (p.waves < kAttnWaves) {
+      p.split_len = p.waves * kSplitLen;
+      return p;
+    }
+  }
+  // Positions per split.  Two waves per SIMD: the most that still gives the GPU
+  // two blocks per CU; longer splits spend fewer prologues and merges (whole
+  // step at 16 x 4096 positions: 94.3 us with 256, 92.7 with 512, 91.4 with 1024;
+  // 128 x 380: 126, 122, 122).  One wave per SIMD: nothing covers a block's
+  // latencies, so the length whose rounds of blocks take least (8 query heads,
+  // 64 pairs x 2048 positions: 25.8 us with the split kernel, 30.8 with 256, 24.7
+  // with 512; 128 x 1250: 32.0, 39.8, 34.4, with 768 30.2).
+  if (one) {
+    for (int len = kMaxSplitLen - kSplitLen; len >= kSplitLen; len -= kSplitLen)
+      if (ring_rounds(max_ctx, heads, len, round) < ring_rounds(max_ctx, heads, p.split_len, round)) p.split_len = len;
+  } else {
+    while (p.split_len > kSplitLen && heads * ((max_ctx + p.split_len - 1) / p.split_len) < round) p.split_len /= 2;
+  }
+  // A short last split goes behind every full one: dealt in turn with them, the
+  // last full ones start late and the launch ends on a few blocks (4 query heads
+  // x 128: 512 pairs x 1100 positions 76.7 us with the split kernel, 79.5 dealt in
+  // turn, 64.9 split-major; 256 x 600: 27.8, 29.2, 24.6; 1 query head x 64: 1024 x 1100 65.7,
+  // 84.1, 61.6).  Else a sequence's splits run side by side (128 x 2500: 40.7
+  // against 42.8; 256 x 5000 positions of 1 query head x 64: 63.0 against 68.0).
+  const int n_split = (max_ctx + p.split_len - 1) / p.split_len;
+  const int last = max_ctx - (n_split - 1) * p.split_len;
+  p.split_major = n_split > 1 && n_split <= 65535 && 4ll * last < 3ll * p.split_len;
+  return p;
+}
+
+template <int D, int G, int W>
+void launch_ring_w(const AttnArgs& a, int B, hipStream_t s) {
+  constexpr int lds = Ring<D, G, W>::kLds;
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(attn_ring_kernel<D, G, W>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  (void)attr;
+  const dim3 grid = a.split_major ? dim3(a.n_head_kv, B, a.n_split) : dim3(a.n_split, a.n_head_kv, B);
+  hipLaunchKernelGGL((attn_ring_kernel<D, G, W>), grid, dim3(W * kWave), lds, s, a);
 }
 
 template <int D, int G>
-void launch_ring_n(const AttnArgs& a, int B, hipStream_t s) {
-  constexpr int lds = Ring<D, G>::kLds;
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(attn_ring_kernel<D, G>),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  (void)attr;
-  hipLaunchKernelGGL((attn_ring_kernel<D, G>), dim3(a.n_split, a.n_head_kv, B), dim3(kAttnThreads), lds, s, a);
+void launch_ring_n(const AttnArgs& a, int waves, int B, hipStream_t s) {
+  if (waves == 1)
+    launch_ring_w<D, G, 1>(a, B, s);
+  else if (waves == 2)
+    launch_ring_w<D, G, 2>(a, B, s);
+  else
+    launch_ring_w<D, G, kAttnWaves>(a, B, s);
 }
 
 template <int D>
-hipError_t launch_ring(const AttnArgs& a, int G, int B, hipStream_t s) {
+hipError_t launch_ring(const AttnArgs& a, int G, int waves, int B, hipStream_t s) {
   switch (G) {
-    case 1: launch_ring_n<D, 1>(a, B, s); break;
-    case 2: launch_ring_n<D, 2>(a, B, s); break;
-    case 4: launch_ring_n<D, 4>(a, B, s); break;
-    case 8: launch_ring_n<D, 8>(a, B, s); break;
+    case 1: launch_ring_n<D, 1>(a, waves, B, s); break;
+    case 2: launch_ring_n<D, 2>(a, waves, B, s); break;
+    case 4: launch_ring_n<D, 4>(a, waves, B, s); break;
+    case 8: launch_ring_n<D, 8>(a, waves, B, s); break;
     default: return hipErrorNotSupported;
   }
   return hipGetLastError();
@@ -915,10 +985,13 @@ hipError_t launch_split_d(const AttnArgs& a, int D, int G, int B, hipStream_t s)
   switch (D) {
     case 16: return launch_split_g<T, 16, 8>(a, G, B, s);
     case 32: return launch_split_g<T, 32, 8>(a, G, B, s);
-    case 64: return launch_split_g<T, 64, kLanesPerPos64>(a, G, B, s);
-    case 128: return launch_split_g<T, 128, kLanesPerPos128>(a, G, B, s);
-    default: return hipErrorNotSupported;
+    default: break;
   }
+  if constexpr (sizeof(T) == 4) {  // bf16: attn_ring_kernel
+    if (D == 64) return launch_split_g<T, 64, kLanesPerPos64>(a, G, B, s);
+    if (D == 128) return launch_split_g<T, 128, kLanesPerPos128>(a, G, B, s);
+  }
+  return hipErrorNotSupported;
 }
 
 }  // namespace
@@ -955,13 +1028,17 @@ hipError_t launch_attn_decode(const float* q_rot, const void* k_pool, const void
   a.scale = scale;
   a.part = part;
   const int G = n_head / n_head_kv;
-  const bool ring = dtype == DT_BF16 && (head_dim == 64 || head_dim == 128) &&
-                    reinterpret_cast<uintptr_t>(k_pool) % 16 == 0 && reinterpret_cast<uintptr_t>(v_pool) % 16 == 0;
-  a.split_len = ring ? ring_split_len(max_ctx, static_cast<int64_t>(batch) * n_head_kv) : kSplitLen;
+  const bool ring = dtype == DT_BF16 && (head_dim == 64 || head_dim == 128);
+  RingPlan plan{kSplitLen, kAttnWaves, false};
+  if (ring) plan = ring_plan(max_ctx, static_cast<int64_t>(batch) * n_head_kv, head_dim, G);
+  a.split_len = plan.split_len;
+  a.split_major = plan.split_major;
   a.n_split = (max_ctx + a.split_len - 1) / a.split_len;  // at most attn_decode_splits(max_ctx)
   if (a.n_split > 0) {
-    const hipError_t e = ring && head_dim == 64 ? launch_ring<64>(a, G, batch, s)
-                         : ring                 ? launch_ring<128>(a, G, batch, s)
+    if (reinterpret_cast<uintptr_t>(k_pool) % 16 || reinterpret_cast<uintptr_t>(v_pool) % 16)
+      return hipErrorInvalidValue;  // 16-byte loads (the entry points check this too)
+    const hipError_t e = ring && head_dim == 64 ? launch_ring<64>(a, G, plan.waves, batch, s)
+                         : ring                 ? launch_ring<128>(a, G, plan.waves, batch, s)
                          : dtype == DT_F32      ? launch_split_d<float>(a, head_dim, G, batch, s)
                                                 : launch_split_d<bf16_t>(a, head_dim, G, batch, s);
     if (e != hipSuccess) return e;

@@ -1,6 +1,6 @@
 """bf16 paged attention with head_dim 64 and 128 (attn_ring_kernel) against the
-oracle, at the edges of its 16-position tiles, 64-position chunks and 256- to
-1024-position splits.
+oracle, at the edges of its 16-position tiles, 64-position chunks, 256- to
+1024-position splits and blocks of 1, 2 and 4 waves.
 
 The output projection is the identity, so the output is the attention itself
 rounded to bf16 once (2^-9 relative); q is carried to about 16 significant
@@ -25,12 +25,24 @@ EDGES = [0, 1, 15, 16, 17, 63, 64, 65, 127, 191, 192, 255, 256, 257, 320, 449, 5
 
 # (lens, n_embd, H, Hkv, block_size): every query group size with both head
 # sizes, block sizes that no tile divides; 64 sequences x 8 heads, whose splits
-# hold 512 and 1024 positions (contexts up to 520 and 1100).
+# hold 512 and 1024 positions (contexts up to 520 and 1100, the short last
+# splits behind the full ones); more than 512 pairs of at most 64 and 128
+# positions (blocks of one and two waves); 8 query heads x 128: more than 256
+# pairs of at most 64 and 300, 1024 of at most 200 (one wave per 256
+# positions), and 128 pairs of 1250, in splits of 768.
 @pytest.mark.parametrize("lens,n_embd,H,Hkv,bs", [
     (EDGES, 128, 1, 1, 16), (EDGES, 128, 2, 1, 5), (EDGES, 256, 4, 1, 32), (EDGES, 512, 8, 1, 7),
     (EDGES, 128, 2, 2, 64), (EDGES, 256, 2, 1, 3), (EDGES, 512, 4, 1, 16), (EDGES, 1024, 8, 1, 1),
     ([520] + [1 + 8 * i for i in range(64)] + [513], 512, 8, 8, 16),
     ([1100, 1025, 1024, 1023, 961, 960, 4] + [17 * i for i in range(57)], 512, 8, 8, 32),
+    ([64, 63, 17, 4] + [i % 65 for i in range(62)], 512, 8, 8, 16),
+    ([64, 1, 0, 33] + [i % 65 for i in range(62)], 1024, 8, 8, 16),
+    ([128, 127, 65, 64] + [2 * i % 129 for i in range(62)], 512, 8, 8, 16),
+    ([128, 64, 0, 66] + [2 * i % 129 for i in range(62)], 2048, 16, 8, 16),
+    ([64, 63, 17, 4] + [i % 65 for i in range(130)], 2048, 16, 2, 16),
+    ([300, 257, 256, 200, 65] + [3 * i % 301 for i in range(125)], 2048, 16, 2, 16),
+    ([200, 65, 64, 129, 193] + [i % 201 for i in range(1020)], 1024, 8, 1, 16),
+    ([1250, 769, 768, 767, 1024] + [20 * i for i in range(59)], 2048, 16, 2, 16),
 ])
 def test_ring_edges(fm, lens, n_embd, H, Hkv, bs):
     rng = np.random.default_rng(len(lens) * n_embd + bs)

@@ -96,6 +96,26 @@ def test_router_f32(fm, wl, T, H, E, k):
     np.testing.assert_allclose(w.cpu().numpy(), rw, rtol=1e-5, atol=1e-7)
 
 
+# The block's router: partial logits of 512-column ranges of the hidden axis,
+# kept in the block's y rows, then the top-k that sums them; on both sides of
+# 64 tokens, with a last range of 16 and 32 columns, 5 ranges, each width of
+# the top-k.  k = 1 with more ranges x experts than hidden columns: the
+# partials do not fit, one kernel routes (up to 128 experts, and beyond).
+@pytest.mark.parametrize("T,H,E,k", [(3, 2064, 64, 6), (64, 528, 65, 4), (65, 2064, 128, 8), (33, 544, 129, 6),
+                                     (64, 2064, 16, 2), (100, 2064, 256, 8), (200, 64, 128, 1), (40, 64, 256, 1)])
+def test_block_router_f32(fm, wl, T, H, E, k):
+    cfg = wl.Config("RB", H, 32, E, k, (T,), "f32", "f32", True, 1e-6, seed=E)
+    x, wr, _ = wl.router_inputs(cfg, T)
+    dev = lambda a: torch.from_numpy(a).cuda()  # noqa: E731
+    up, gate, down = (torch.zeros(s, device="cuda") for s in ((32, H, E), (32, H, E), (H, 32, E)))
+    block = fm.MoEFFNBlock(dev(wr), up, gate, down, E, k, H, 32, True, act_dtype=torch.float32)
+    block(dev(x))
+    ids, w = block.routing()[:2]
+    rids, rw = om.router(x, wr, k, True)
+    np.testing.assert_array_equal(ids.cpu().numpy(), rids)
+    np.testing.assert_allclose(w.cpu().numpy(), rw, rtol=1e-5, atol=1e-7)
+
+
 # Attention projections: one expert's rows in order, K split into partials.
 @pytest.mark.parametrize("B,n_embd,H,Hkv", [(1, 128, 2, 1), (16, 512, 4, 2), (65, 1024, 8, 8), (130, 256, 16, 2)])
 def test_attention_projections_f32(fm, B, n_embd, H, Hkv):

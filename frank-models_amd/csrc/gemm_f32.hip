@@ -12,7 +12,13 @@
 // pair per 16 inputs with no load in flight across them.  Measured
 // (DeepSeek-V2-Lite in fp32, 64 experts x 2048 x 1408, top-6): 500 tokens
 // gate/up 1607 -> 405-440 us (86 TFLOP/s, 3.6 TB/s) and down 1059 -> 202-224
-// us; 64 tokens, whole block, 378 us (5.9 TB/s of weights).
+// us; 64 tokens, whole block, 378 us (5.9 TB/s of weights).  Other shapes, whole
+// block, SIMT kernel -> this one (hidden x ff, experts, top-k): 512 x 1792, 8, 2
+// with 1 / 40 / 2000 tokens 300 / 347 / 857 -> 40 / 51 / 270 us; 2048 x 768, 128, 8
+// with 1 / 100 / 500 tokens 619 / 3171 / 4439 -> 60 / 217 / 600; 4096 x 14336, 8, 2
+// with 1 / 64 tokens 2842 / 6066 -> 328 / 1033.  Counters at 500 tokens: the
+// matrix cores are busy 66% (gate/up) and 60% (down) of the time, 15% of it on
+// padding rows, beside 3.7 TB/s from HBM: neither bound is reached alone.
 //
 // Block: 256 threads, a tile of BM assignment rows x 32 * WN weight rows,
 // stages of KS inputs through a ring in LDS filled by global_load_lds (16
@@ -315,6 +321,7 @@ int col_tiles(const GroupedGemmArgs& g, int wn) {
   return static_cast<int>((g.N + cols - 1) / cols);
 }
 
+// (The lines of pick_bm, pick_wn and launch_tile are DeepSeek-V2-Lite's.)
 // Rows per tile: 32 up to 20 rows per expert on average, where a narrower
 // token part leaves LDS for more blocks, else 64, which streams the weights
 // once for more rows.  Measured (DeepSeek-V2-Lite in fp32, whole block,

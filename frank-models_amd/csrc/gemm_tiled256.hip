@@ -878,6 +878,10 @@ __device__ __forceinline__ WaveCtx tile_ctx(const GroupedGemmArgs& g, const Tile
 // activations 100 tokens 304 -> 286 us; on thin last tiles too, the gate
 // projection at Mixtral's 250 rows per expert went 418 -> 456 us, and the main
 // loop's stages lose far more (Mixtral 4096 tokens 2345 -> 2618 us).
+// A call repeated on weights that the infinity cache still holds loses by it: 16
+// experts of 1024 x 2816 (138 MB), 300 tokens, before the narrow loop -> now, 97 ->
+// 103 us repeated, 106 -> 101 cold; in a model the other layers' weights pass
+// between two calls of one layer.
 constexpr int kNarrowRows = 128;
 
 template <int MG>
